@@ -328,6 +328,9 @@ static double tile_flops(const GemmTask& g)
 
 static const int SMALL_M = 64;   // fronts with m <= 64 run whole in one wave
 static const int NB = 64;        // panel block width of large fronts
+// elements behind the L arena: k_gemm_tile128 loads 16 bytes from the last
+// row of a column on (3 elements past it in FP32, 1 in FP64)
+static const long long L_SPARE = 4;
 
 // One independent system of a (possibly batched) device schedule.
 struct SysView {
@@ -1139,7 +1142,7 @@ extern "C" long long taucs_amd_factor_device_bytes(void* vL, int precision, int 
   const long long elem = precision == TAMD_PREC_FP64 ? 8 : 4;
   const long long n = F->n, cap = std::max(nrhs, 16);
   long long b = (long long)D.struct_bytes + sizeof(int);
-  b += elem * (std::max(D.L_elems, 1LL) + std::max(D.U_elems, 1LL) + std::max(D.I_elems, 1LL));
+  b += elem * (std::max(D.L_elems, 1LL) + L_SPARE + std::max(D.U_elems, 1LL) + std::max(D.I_elems, 1LL));
   b += elem * (D.W_per_rhs * cap + n * cap + 64LL * 16 * std::max(D.part_slots, 1LL));
   b += (long long)sizeof(int) * (D.sync_n + 1);
   b += 2LL * 8 * n * std::max(nrhs, 1);
@@ -1338,7 +1341,7 @@ static int launch_numeric(tamd_dev* D, Emitter& E, bool bf16upd, bool prof)
           EMIT(lane, join, k_gemm_tile_bf16, dim3(op.count), dim3(256),
                (const GemmTask*)(D->d_gemm + op.start), (const float*)L, (float*)L, (float*)U);
         else if (op.tile == 128)
-          EMIT(lane, join, k_gemm_tile128<T>, dim3(op.count), dim3(512),
+          EMIT(lane, join, k_gemm_tile128<T>, dim3(op.count), dim3(256),
                (const GemmTask*)(D->d_gemm + op.start), (const T*)L, L, U);
         // the latency-shaped tile (the same bits) where each workgroup has a
         // CU to itself: K <= 64, or a main-chain launch of at most
@@ -1479,7 +1482,7 @@ static int ensure_numeric_buffers(tamd_factor* F)
   int elem = prec == TAMD_PREC_FP64 ? 8 : 4;
   if (D->prec != prec) {
     tamd_dev_free_numeric(F);
-    if (dev_malloc(&D->L, (size_t)elem * (D->L_elems > 0 ? D->L_elems : 1)) != 0
+    if (dev_malloc(&D->L, (size_t)elem * ((D->L_elems > 0 ? D->L_elems : 1) + L_SPARE)) != 0
         || dev_malloc(&D->U, (size_t)elem * (D->U_elems > 0 ? D->U_elems : 1)) != 0
         || dev_malloc(&D->Inv, (size_t)elem * (D->I_elems > 0 ? D->I_elems : 1)) != 0) {
       tamd_dev_free_numeric(F);

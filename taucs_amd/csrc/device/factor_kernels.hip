@@ -4,6 +4,7 @@
 // Reference computation per front (src/taucs_sn_llt.c:1086-1194): assemble
 // A's columns into [F1;F2], dpotrf F1, dtrsm F2 <- F2 L11^-T, dsyrk
 // U <- U - F2 F2^T; then extend-add U into the parent (:1200-1240).
+#include <type_traits>
 #include "kernels.h"
 
 namespace tamd {
@@ -1902,108 +1903,193 @@ __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict
   potrf_mw_block<T>(fr, PanelTask{t.pf_front, t.pf_k0, t.Md, 0, 0}, L, Inv, info, fallback, smem);
 }
 
-// 128 x 128 tile for the large trailing updates and SYRKs: 8 waves (2 x 4),
-// each a 64 x 32 sub-tile of 4 x 2 MFMA blocks.  A 64 x 64 sub-tile per wave
-// (4 waves) reuses each LDS fragment more, but its 128 accumulator registers
-// leave room for two waves per SIMD only; with 64 x 32 four waves share a
-// SIMD and keep its MFMA pipe busier (measured on a K = 512 trailing update
-// of a 6144-row front: 45.0 against 37.9 TFLOP/s FP64, the same bits).  K is
-// staged in chunks of 16 with the next chunk prefetched into registers.
-// Same task format (M, N <= 128) and epilogue as the 64 x 64 tile.
-#define TK2 16
-#define TPAD2 4
+// 128 x 128 tile for the large trailing updates and SYRKs: 4 waves (2 x 2),
+// each a 64 x 64 sub-tile of 4 x 4 MFMA blocks, two workgroups to a CU.  The
+// FP64 MFMA takes 64 cycles and a wave can issue other instructions behind it,
+// so what bounds the tile is any stretch in which a wave issues something else
+// for longer than that.  The chunk (16 columns of K in FP64, 32 in FP32; two
+// LDS buffers, one barrier) is therefore laid out by hand, one operation
+// behind each MFMA: the fragments of the next step, the next chunk's stores
+// into the other buffer and, as each store frees its registers, the loads of
+// the chunk after it (a whole chunk ahead, 16 bytes a lane).  The barrier
+// comes before the last step, whose fragments are in registers by then, and
+// the next chunk's first fragments are read behind that step's MFMAs.  Only
+// the chunk that holds the end of K zeroes entries: the selects cost 8% of the
+// loop when every chunk had them.  Measured against eight waves of 64 x 32
+// sub-tiles with one LDS buffer and two barriers per chunk, TFLOP/s, FP64 /
+// FP32: 16K rows, K = 512, lower triangle 54 -> 62 / 87 -> 112; 6144 rows,
+// K = 256 43 -> 48 / 71 -> 88.
+// A workgroup in an odd wave slot of its SIMD runs at a raised priority, so
+// that two workgroups of a CU drift apart and one's loads and stores of C
+// meet the other's products (K = 256: 45 -> 47 TFLOP/s).
+// The MFMA steps take k = 16 c + 4 (lane / 16) + step, the order of the
+// 64 x 64 tile: the results are bitwise the same.
+// C goes through a buffer resource: entries outside the tile (or above a
+// diagonal tile's diagonal) get an offset past its end, where loads return 0
+// and stores are dropped.  The 16-byte loads may read up to 3 elements past
+// the last row of a column (rows that are not stored); the L arena ends with
+// as many spare elements.
+typedef unsigned u2_t __attribute__((ext_vector_type(2)));
 template <typename T>
-__global__ __launch_bounds__(512) void k_gemm_tile128(const GemmTask* __restrict__ tasks,
-                                                      const T* Lsrc, T* L, T* U)
+__global__ __launch_bounds__(256, 2) void k_gemm_tile128(const GemmTask* __restrict__ tasks,
+                                                         const T* Lsrc, T* L, T* U)
 {
   typedef typename Mfma<T>::acc_t acc_t;
-  __shared__ T As[TK2][128 + TPAD2];
-  __shared__ T Bs[TK2][128 + TPAD2];
+  constexpr int VEC = 16 / (int)sizeof(T);      // rows of one load
+  constexpr int KC = 128 / (int)sizeof(T);      // columns of a chunk
+  constexpr int NS = KC / 4;                    // MFMA steps of a chunk
+  constexpr int RG = 128 / VEC, KL = 256 / RG;  // loader: row groups, columns at a time
+  constexpr int NQ = KC / KL;                   // loads per operand and thread (4)
+  constexpr int LDR = 132;                      // the four lane groups of a fragment read
+                                                // fall into different banks
+  typedef T vec_t __attribute__((ext_vector_type(VEC)));
+  typedef vec_t vecu_t __attribute__((aligned(sizeof(T))));
+  __shared__ __align__(16) T As[2 * KC * LDR];
+  __shared__ __align__(16) T Bs[2 * KC * LDR];
+  // HW_ID, wave slot within the SIMD
+  if (__builtin_amdgcn_s_getreg(0x1804) & 1) __builtin_amdgcn_s_setprio(1);
   const GemmTask t = tasks[blockIdx.x];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = (wave >> 2) * 64, wc = (wave & 3) * 32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
+  const int c16 = lane & 15, g = lane >> 4;
   const T* A = Lsrc + t.a_off;
   const T* B = Lsrc + t.b_off;
-  acc_t acc[4][2];
+  acc_t acc[4][4];
 #pragma unroll
   for (int a = 0; a < 4; a++)
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[a][b][r] = (T)0;
 
-  const int li = tid & 127, lk = tid >> 7;  // loader: row li, k = lk + 4q
-  T ra[TK2 / 4], rb[TK2 / 4];
-  auto fetch = [&](int kc) {
+  const int lr = (tid % RG) * VEC, lk = RG == 64 ? wave : tid / RG;
+  const int lam = min(lr, t.M - 1), lbn = min(lr, t.N - 1), K1 = t.K - 1;
+  vec_t ra[NQ], rb[NQ];
+  T* const sA = As + lk * LDR + lr;
+  T* const sB = Bs + lk * LDR + lr;
+  auto fetch = [&](int q, int kc) {  // clamped to the last column
+    const long long o = (long long)min(kc + lk + KL * q, K1) * t.ld;
+    ra[q] = *(const vecu_t*)(A + o + lam);
+    rb[q] = *(const vecu_t*)(B + o + lbn);
+  };
+  // TAIL: columns past K become zero
+  auto stash = [&](int q, int buf, int kc, auto TAIL) {
+    asm volatile("" : "+v"(ra[q]));
+    asm volatile("" : "+v"(rb[q]));
+    vec_t va = ra[q], vb = rb[q];
+    if constexpr (decltype(TAIL)::value) {
+      const bool kin = kc + lk + KL * q <= K1;
 #pragma unroll
-    for (int q = 0; q < TK2 / 4; q++) {
-      const int k = kc + lk + 4 * q;
-      const bool kin = k < t.K;
-      ra[q] = (kin && li < t.M) ? A[li + (long long)k * t.ld] : (T)0;
-      rb[q] = (kin && li < t.N) ? B[li + (long long)k * t.ld] : (T)0;
+      for (int e = 0; e < VEC; e++) {
+        va[e] = kin ? va[e] : (T)0;
+        vb[e] = kin ? vb[e] : (T)0;
+      }
+    }
+    *(vec_t*)(sA + (buf * KC + KL * q) * LDR) = va;
+    *(vec_t*)(sB + (buf * KC + KL * q) * LDR) = vb;
+  };
+  T fa[2][4], fb[2][4];
+  // fragment m of step s: A rows for m < 4, B rows for the others
+  auto frag = [&](int s, int buf, int m) {
+    const int kr = (buf * KC + 16 * (s >> 2) + 4 * g + (s & 3)) * LDR + c16;
+    if (m < 4) fa[s & 1][m] = As[kr + wr + 16 * m];
+    else fb[s & 1][m - 4] = Bs[kr + wc + 16 * (m - 4)];
+  };
+  // the 16 MFMAs of a step, op(m) behind the m-th
+  auto step = [&](int s, auto&& op) {
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      acc[m >> 2][m & 3] = Mfma<T>::step(fb[s & 1][m & 3], fa[s & 1][m >> 2], acc[m >> 2][m & 3]);
+      __builtin_amdgcn_sched_barrier(0);
+      op(m);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  fetch(0);
-  for (int kc = 0; kc < t.K; kc += TK2) {
+  // chunk ch; NEXT: the next chunk is in registers, NEXT2: the one after it
+  // is to be loaded
+  auto chunk = [&](int ch, auto NEXT, auto NEXT2) {
+    constexpr bool next = decltype(NEXT)::value, next2 = decltype(NEXT2)::value;
+    const std::integral_constant<bool, next && !next2> TAIL{};
+    const int buf = ch & 1, kc1 = (ch + 1) * KC, kc2 = kc1 + KC;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < TK2 / 4; q++) {
-      As[lk + 4 * q][li] = ra[q];
-      Bs[lk + 4 * q][li] = rb[q];
-    }
+    for (int s = 0; s < NS - 1; s++)
+      step(s, [&](int m) {
+        if (m < 8) frag(s + 1, buf, m);
+        if (s < 2 && next && (m == 8 || m == 12)) stash(2 * s + (m - 8) / 4, buf ^ 1, kc1, TAIL);
+        if (s < 2 && next2 && (m == 10 || m == 14)) fetch(2 * s + (m - 10) / 4, kc2);
+      });
+    // this chunk's fragments are all read and the next chunk is stored
     __syncthreads();
-    if (kc + TK2 < t.K) fetch(kc + TK2);
+    __builtin_amdgcn_sched_barrier(0);
+    step(NS - 1, [&](int m) {
+      if (next && m < 8) frag(0, buf ^ 1, m);
+    });
+  };
+  const std::true_type Y{};
+  const std::false_type N{};
+  const int nch = (t.K + KC - 1) / KC;
 #pragma unroll
-    for (int kk = 0; kk < TK2; kk += 4) {
-      const int kr = kk + (lane >> 4), c16 = lane & 15;
-      T af[4], bf[2];
+  for (int q = 0; q < NQ; q++) fetch(q, 0);
 #pragma unroll
-      for (int a = 0; a < 4; a++) af[a] = As[kr][wr + 16 * a + c16];
+  for (int q = 0; q < NQ; q++) stash(q, 0, 0, Y);
 #pragma unroll
-      for (int b = 0; b < 2; b++) bf[b] = Bs[kr][wc + 16 * b + c16];
+  for (int q = 0; q < NQ; q++) fetch(q, KC);
+  __syncthreads();
 #pragma unroll
-      for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = Mfma<T>::step(bf[b], af[a], acc[a][b]);
-    }
-    __syncthreads();
-  }
+  for (int m = 0; m < 8; m++) frag(0, 0, m);
+  int ch = 0;
+  for (; ch + 2 < nch; ch++) chunk(ch, Y, Y);
+  if (ch + 1 < nch) chunk(ch++, Y, N);
 
-  // C -= acc, eight entries a lane at a time with their loads in flight
-  // together (clamped to the tile, dropped outside it; the empty asm keeps
-  // the compiler from sinking each load into its store's condition; eight
-  // keep the kernel within the 128 registers of four waves per SIMD)
+  // C -= acc; the first 16 entries of a lane are loaded behind the last
+  // chunk's MFMAs, the others one row block ahead of their use
   T* C = ((t.flags & 1) ? U : L) + t.c_off;
   const bool diag = (t.flags & 2) != 0;
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(C, 0, 0x7fffffff, 0x00020000);
+  constexpr int ES = (int)sizeof(T), RS = sizeof(T) == 8 ? 4 : 1;
+  const int g0 = sizeof(T) == 8 ? g : 4 * g;  // column of (b, r): wc + 16 b + RS r + g0
+  const int vo = (g0 * t.ldc + wr + c16) * ES;
+  T cv[2][4][4];
+  auto cload = [&](int a) {
+    const int im = wr + 16 * a + c16 < t.M ? vo : -1;
 #pragma unroll
-  for (int a0 = 0; a0 < 4; a0++) {
-    T cv[1][2][4];
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-    for (int a = 0; a < 1; a++)
+      for (int r = 0; r < 4; r++) {
+        const int j = wc + 16 * b + RS * r;
+        const int v = j + g0 < t.N ? im : -1, so = (j * t.ldc + 16 * a) * ES;
+        if constexpr (sizeof(T) == 8)
+          cv[a & 1][b][r] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, v, so, 0));
+        else
+          cv[a & 1][b][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, v, so, 0));
+      }
+  };
+  auto cstore = [&](int a) {
+    const int i = wr + 16 * a + c16, im = i < t.M ? vo : -1;
+    const int jm = diag ? min(t.N, i + 1) : t.N;
 #pragma unroll
-      for (int b = 0; b < 2; b++)
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int i = min(wr + (a0 + a) * 16 + (lane & 15), t.M - 1);
-          const int j = min(wc + b * 16 + Mfma<T>::drow(lane, r), t.N - 1);
-          cv[a][b][r] = C[i + (long long)j * t.ldc];
-        }
+      for (int r = 0; r < 4; r++) {
+        const int j = wc + 16 * b + RS * r;
+        const int v = j + g0 < jm ? im : -1, so = (j * t.ldc + 16 * a) * ES;
+        const T w = cv[a & 1][b][r] - acc[a][b][r];
+        if constexpr (sizeof(T) == 8)
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2_t, w), rs, v, so, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, w), rs, v, so, 0);
+      }
+  };
+  cload(0);
+  __builtin_amdgcn_sched_barrier(0);
+  chunk(ch, N, N);
 #pragma unroll
-    for (int a = 0; a < 1; a++)
-#pragma unroll
-      for (int b = 0; b < 2; b++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) asm volatile("" : "+v"(cv[a][b][r]));
-#pragma unroll
-    for (int a = 0; a < 1; a++)
-#pragma unroll
-      for (int b = 0; b < 2; b++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int i = wr + (a0 + a) * 16 + (lane & 15);
-          const int j = wc + b * 16 + Mfma<T>::drow(lane, r);
-          if (i < t.M && j < t.N && (!diag || i >= j))
-            C[i + (long long)j * t.ldc] = cv[a][b][r] - acc[a0 + a][b][r];
-        }
+  for (int a = 0; a < 4; a++) {
+    if (a + 1 < 4) cload(a + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    cstore(a);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 

@@ -240,3 +240,31 @@ def test_matrix_file_through_the_drop_in(tmp_path):
         assert np.abs(x - xd).max() <= 1e-10 * np.abs(xd).max()
     L.free()
     F.free()
+
+
+@pytest.mark.parametrize("prec", [T.FP64, T.FP32])
+@pytest.mark.parametrize("dims,width", [((52, 50, 47), 256), ((50, 51, 53), 192)])
+def test_tile_edges_give_the_same_bits(prec, dims, width):
+    """The 128 x 128 tiles take K in the 64 x 64 tiles' order, so a factor does
+    not depend on which of the two a launch uses.  The boxes' fronts have row
+    counts, update orders and depths K (the SYRKs' K = s, and 192 against the
+    chunks of 16 and 32 columns) that are no multiples of a tile or a chunk."""
+    print(f"case: tile edges bitwise, mesh3d {dims}, width {width}, precision {prec}", flush=True)
+    A = T.mesh3d(*dims)
+    perm, inv = T.order(A, "genmmd")
+    PA = T.permute(A, perm, inv)
+    digests, wide = [], []
+    try:
+        T.lib.taucs_amd_set_panel_width(width)
+        for tile in (64, 128):
+            T.lib.taucs_amd_set_gemm_tile(tile)
+            F = T.factor_symbolic(PA)
+            assert F.numeric(PA, prec) == 0
+            digests.append(F.digest())
+            wide.append(int((F.op_profile()["tile"] == 128).sum()))
+            F.free()
+    finally:
+        T.lib.taucs_amd_set_panel_width(256)
+        T.lib.taucs_amd_set_gemm_tile(64)
+    assert wide[0] == 0 and wide[1] > 0
+    assert digests[0] == digests[1]
