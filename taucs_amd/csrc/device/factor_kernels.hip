@@ -254,11 +254,12 @@ __device__ __forceinline__ float rlane<float>(float v, int l)
 }
 
 // d = sqrt(p) and rd = 1/d for a pivot p > 0.  FP32: correctly rounded.
-// FP64: Newton's iteration for y = 1/sqrt(p), y <- y + y (1 - p y^2) / 2,
-// twice from the hardware estimate (each step squares the relative error),
-// then d = p y corrected once by the same iteration for sqrt,
-// d <- d + y (p - d^2) / 2.  Both end within about one ulp, and the chain is
-// half as long as a correctly rounded sqrt followed by a division: the pivot
+// FP64: y = 1/sqrt(p) from the hardware estimate (relative error 2^-26) by one
+// third-order step, y <- y (1 + h/2 + 3 h^2/8) with h = 1 - p y^2, then d = p y
+// corrected once by Newton's iteration for sqrt, d <- d + y (p - d^2) / 2.
+// Over 2^20 pivots of 40 decades rd is within 0.98 ulp (two Newton steps: 0.99)
+// and d within 0.50; the chain is two operations shorter than with two Newton
+// steps, and half as long as a correctly rounded sqrt and a division: the pivot
 // step is the latency of the whole block.
 template <typename T>
 __device__ __forceinline__ void sqrt_pair(T p, T& d, T& rd)
@@ -266,17 +267,17 @@ __device__ __forceinline__ void sqrt_pair(T p, T& d, T& rd)
   d = sqrt(p);
   rd = (T)1 / d;
 }
+__device__ __forceinline__ double rsqrt_step(double p, double y)
+{
+  const double h = __builtin_fma(-(p * y), y, 1.0);
+  return __builtin_fma(y * h, __builtin_fma(0.375, h, 0.5), y);
+}
 template <>
 __device__ __forceinline__ void sqrt_pair<double>(double p, double& d, double& rd)
 {
-  double y = __builtin_amdgcn_rsq(p);
-  double h = __builtin_fma(-p * y, y, 1.0);
-  y = __builtin_fma(0.5 * y, h, y);
-  h = __builtin_fma(-p * y, y, 1.0);
-  y = __builtin_fma(0.5 * y, h, y);
-  const double s = p * y;
-  d = __builtin_fma(0.5 * y, __builtin_fma(-s, s, p), s);
-  rd = y;
+  rd = rsqrt_step(p, __builtin_amdgcn_rsq(p));
+  const double s = p * rd;
+  d = __builtin_fma(0.5 * rd, __builtin_fma(-s, s, p), s);
 }
 
 __device__ __forceinline__ void wave_lds_fence()
@@ -514,22 +515,23 @@ __global__ __launch_bounds__(64) void k_potrf_wave(const FrontDesc* __restrict__
   if (lane == 0 && bad) atomicOr(info, 1);
 }
 
-// The diagonal block of a panel step by four waves (256 threads).  The
-// one-wave kernel above is bound by its instruction stream: one wave issues
-// every pivot's chain (broadcast, square root, scaling) and all 2016 rank-1
-// FMAs, so FP32 runs no faster than FP64.  Here the block lives in LDS
-// (column-major, A(i, c) at A[c*PM_LDA + i]) and is factored in 16-column
-// panels: wave 0 factors panel p in registers (lane = row, its 16 panel
-// entries; pivot by lane broadcast and sqrt_pair, the panel's own updates
-// with the multipliers broadcast by readlane), then all four waves apply the
-// panel to the 16 x 16 blocks right of it as rank-16 MFMA updates,
-// C -= L_Qp L_Rp^T.  The inverse X = L^{-1} follows in the same LDS block,
-// transposed into its upper triangle: the four 16 x 16 diagonal blocks by
-// substitution (one wave, lane = (block, column)), then the off-diagonal
-// blocks by distance on MFMA, X_ij = -X_ii sum_k L_ik X_kj, one block per
-// wave.  Loads and stores go through LDS, coalesced.  The MFMA steps apply
-// their products as one fused multiply-add after another in k order, so L
-// and the inverse are bitwise those of k_potrf_wave.
+// The diagonal block of a panel step by four waves (256 threads), in LDS
+// (column-major, A(i, c) at A[c*PM_LDA + i]).  What bounds it is latency: the
+// chain of 64 pivots (broadcast, reciprocal square root, scaling, the column's
+// updates: 190 to 260 cycles each), then the inverse.  So wave 0 runs
+// the chain alone, in 16-column panels (pm_panel), and the other waves do
+// everything else beside it: the updates of the blocks that the next panel
+// does not touch, and the rows of the inverse X = L^{-1} as far as L is
+// known.  Only the next panel's blocks are updated between two panels
+// (rank-16 MFMA updates, one block per wave), and after the last panel only
+// its own block of X and one product per block of X's last row are left.
+// L stays in the lower triangle; X, transposed, in the strict upper one
+// (X(r, c) at A[r*PM_LDA + c], r > c), its diagonal is rdiag.
+// Measured on one block, 64 columns, launch included: FP64 18.3 -> 13.7 us,
+// FP32 18.3 -> 15.9 us, against panels whose multipliers all came by readlane
+// and an inverse after the last panel.
+// The MFMA steps apply their products as one fused multiply-add after another
+// in k order, so L and the inverse are bitwise those of k_potrf_wave.
 #define PM_LDA 65
 
 // C(Q, R) -= L(Q, p) L(R, p)^T on 16 x 16 blocks of A, by one wave; on a
@@ -556,22 +558,218 @@ __device__ __forceinline__ void pm_block_update(T* A, int Q, int R, int p, int l
   }
 }
 
+// Broadcast within each 16 lanes as an operand (DPP row_newbcast, the one DPP
+// control that FP64 has).  A DPP operand must have been written two wait
+// states before, which the compiler does not see in an asm statement: the
+// first broadcast of a value waits itself (FIRST), and the later ones name the
+// first one's result as an operand, so that none can move ahead of it.
+// lane N of the 16
+template <int N>
+__device__ __forceinline__ double bcast16(double v)
+{
+  double d;
+  asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+      : "=v"(d) : "v"(v), "n"(N));
+  return d;
+}
+template <int N>
+__device__ __forceinline__ float bcast16(float v)
+{
+  float d;
+  asm("s_nop 1\n\tv_mov_b32_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+      : "=v"(d) : "v"(v), "n"(N));
+  return d;
+}
+// c - (lane N of v) x, one rounding
+template <int N>
+__device__ __forceinline__ void fms_bcast16_first(double& c, double v, double x)
+{
+  asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+v"(c) : "v"(v), "v"(x), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void fms_bcast16_first(float& c, float v, float x)
+{
+  asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+v"(c) : "v"(v), "v"(x), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void fms_bcast16(double& c, double v, double x, double first)
+{
+  asm("v_fmac_f64_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+v"(c) : "v"(v), "v"(x), "n"(N), "v"(first));
+}
+template <int N>
+__device__ __forceinline__ void fms_bcast16(float& c, float v, float x, float first)
+{
+  asm("v_fmac_f32_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+v"(c) : "v"(v), "v"(x), "n"(N), "v"(first));
+}
+// f(B), .., f(E - 1) with the index a constant
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+
+// Panel p (columns 16p .. 16p+15) by one wave.  Every 16 lanes hold a copy of
+// the panel's diagonal block (lane li its row li), and with SUB each lane also
+// the row `lane` of the whole panel: the pivot and a column's multipliers are
+// then operands broadcast within the 16 lanes, and nothing of a step waits
+// for a scalar register (27 cycles after a readlane) or for LDS.  A dependent
+// FP64 operation takes 5 cycles, so the panel is bound by the instructions it
+// issues (about 6 cycles apiece from a single wave).  The pivots are collected, one a lane; the diagonal, its reciprocals
+// and the checks follow for all 16 at once.  Nothing reads the entries above
+// the diagonal, which hold no defined values.  `mid`: the barrier halfway, at
+// which the other waves hand over within this panel's time.  (A nonpositive
+// pivot's NaNs or infinities run on through a factor that is reported as
+// failed.)
+template <typename T, bool SUB>
+__device__ __forceinline__ void pm_panel(T* A, T* rdiag, const T* dg, int p, int lane, bool mid,
+                                         bool& bad, bool& grow)
+{
+  const int c0 = 16 * p, li = lane & 15;
+  T* const Ac = A + c0 * PM_LDA;
+  T r[16], rs[16], P = (T)1;
+#pragma unroll
+  for (int c = 0; c < 16; c++) {
+    r[c] = Ac[c * PM_LDA + c0 + li];
+    if (SUB) rs[c] = Ac[c * PM_LDA + lane];
+  }
+  static_for<0, 16>([&](auto Q) {
+    constexpr int q = Q;
+    if (q == 8 && mid) __syncthreads();
+    P = li == q ? r[q] : P;
+    const T pv = bcast16<q>(r[q]);
+    T dk, rdk;
+    if constexpr (sizeof(T) == 8) rdk = rsqrt_step(pv, __builtin_amdgcn_rsq(pv));
+    else sqrt_pair(pv, dk, rdk);
+    const T l = r[q] * rdk;
+    const T ls = SUB ? rs[q] * rdk : l;
+    if constexpr (q < 15) {
+      fms_bcast16_first<q + 1>(r[q + 1], l, l);
+      static_for<q + 2, 16>([&](auto J) { fms_bcast16<J>(r[J], l, l, r[q + 1]); });
+      if (SUB) static_for<q + 1, 16>([&](auto J) { fms_bcast16<J>(rs[J], l, ls, r[q + 1]); });
+    }
+    Ac[q * PM_LDA + (SUB ? lane : c0 + li)] = ls;
+  });
+  T d, rd;
+  sqrt_pair(P, d, rd);
+  if (lane < 16) {
+    rdiag[c0 + li] = rd;
+    Ac[li * PM_LDA + c0 + li] = d;
+  }
+  bad = bad || __ballot(!(P > (T)0)) != 0;
+  if constexpr (sizeof(T) == 4) grow = grow || __ballot(P < (T)GROW_TAU * dg[c0 + li]) != 0;
+}
+
+// X_bb = L_bb^{-1} of a 16 x 16 diagonal block by one wave, lane c16 holding
+// column c16: x_i = (delta_ic - sum_t l_it x_t) / l_ii, the even and the odd t
+// summed apart; column by column, so that x_t waits only for x_{t-1}, with
+// column t of L one entry a lane and its entries broadcast.  The entries below
+// the diagonal go to the transposed position; a lane without one stores into
+// `dump` (16 values)
+template <typename T>
+__device__ __forceinline__ void pm_inv_diag(T* A, const T* rdiag, T* dump, int b, int lane)
+{
+  const int c16 = lane & 15;
+  T* const Ab = A + (16 * b) * PM_LDA + 16 * b;
+  T s[2][16], x[16], lc[16];
+#pragma unroll
+  for (int t = 0; t < 15; t++) lc[t] = Ab[t * PM_LDA + c16];
+  const T rd = rdiag[16 * b + c16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    s[0][i] = i == c16 ? (T)1 : (T)0;
+    s[1][i] = (T)0;
+  }
+  static_for<0, 16>([&](auto TT) {
+    constexpr int t = TT;
+    x[t] = (s[0][t] + s[1][t]) * bcast16<t>(rd);
+    if constexpr (t < 15) {
+      fms_bcast16_first<t + 1>(s[t & 1][t + 1], lc[t], x[t]);
+      static_for<t + 2, 16>([&](auto I) { fms_bcast16<I>(s[t & 1][I], lc[t], x[t], s[t & 1][t + 1]); });
+    }
+  });
+  T* const to = Ab + c16;
+#pragma unroll
+  for (int i = 1; i < 16; i++) *(i > c16 ? to + i * PM_LDA : dump + c16) = x[i];
+}
+
+// S_ij = sum_{k=j}^{i-1} L_ik X_kj by one wave, in the accumulator layout
+template <typename T>
+__device__ __forceinline__ typename Mfma<T>::acc_t pm_inv_sum(const T* A, const T* rdiag, int i, int j,
+                                                              int lane)
+{
+  const int c16 = lane & 15, g = lane >> 4;
+  typename Mfma<T>::acc_t acc;
+#pragma clang loop unroll(full)
+  for (int e = 0; e < 4; e++) acc[e] = (T)0;
+  for (int k = j; k < i; k++)
+#pragma clang loop unroll(full)
+    for (int st = 0; st < 4; st++) {
+      const int kr = 4 * st + g;
+      const T a = A[(16 * k + kr) * PM_LDA + 16 * i + c16];
+      T x = A[(16 * k + kr) * PM_LDA + 16 * j + c16];
+      if (k == j) x = kr > c16 ? x : kr == c16 ? rdiag[16 * j + c16] : (T)0;
+      acc = Mfma<T>::step(a, x, acc);
+    }
+  return acc;
+}
+
+// X_ij = -X_ii S_ij by one wave (ts: its 16 x 17 staging tile)
+template <typename T>
+__device__ __forceinline__ void pm_inv_block(T* A, const T* rdiag, T* ts, int i, int j,
+                                             const typename Mfma<T>::acc_t& S, int lane)
+{
+  const int c16 = lane & 15, g = lane >> 4;
+#pragma clang loop unroll(full)
+  for (int e = 0; e < 4; e++) ts[Mfma<T>::drow(lane, e) * 17 + c16] = S[e];
+  wave_lds_fence();
+  typename Mfma<T>::acc_t xr;
+#pragma clang loop unroll(full)
+  for (int e = 0; e < 4; e++) xr[e] = (T)0;
+#pragma clang loop unroll(full)
+  for (int st = 0; st < 4; st++) {
+    const int kr = 4 * st + g;
+    const T v = A[(16 * i + c16) * PM_LDA + 16 * i + kr];
+    const T a = c16 > kr ? v : c16 == kr ? rdiag[16 * i + c16] : (T)0;
+    xr = Mfma<T>::step(a, ts[kr * 17 + c16], xr);
+  }
+#pragma clang loop unroll(full)
+  for (int e = 0; e < 4; e++) A[(16 * i + Mfma<T>::drow(lane, e)) * PM_LDA + 16 * j + c16] = -xr[e];
+  wave_lds_fence();
+}
+
 // LDS of potrf_mw_block, in bytes: the block A (64 x PM_LDA), rdiag, dg, the
 // four waves' 16 x 17 staging tiles Ts, and one flag
 template <typename T>
 constexpr int potrf_mw_lds() { return (int)sizeof(T) * (64 * PM_LDA + 64 + 64 + 4 * 16 * 17) + 16; }
 
+// entry (i, j) of the block as potrf_mw_block wants it in LDS: the lower
+// triangle of its kb x kb, the identity beyond
 template <typename T>
+__device__ __forceinline__ void pm_stage(T* A, T* dg, int i, int j, int kb, T v)
+{
+  if (!(i < kb && j < kb && i >= j)) v = i == j ? (T)1 : (T)0;
+  A[j * PM_LDA + i] = v;
+  if (i == j) dg[i] = v;
+}
+
+// STAGED: the caller has put the block into A and dg (pm_stage), and has
+// stored it in the panel too in FP32, for the FP64 fallback
+template <typename T, bool STAGED>
 __device__ __forceinline__ void potrf_mw_block(const FrontDesc* __restrict__ fr, const PanelTask t,
                                                T* __restrict__ L, T* __restrict__ Inv,
                                                int* __restrict__ info, int fallback,
                                                unsigned char* smem)
 {
   typedef typename Mfma<T>::acc_t acc_t;
-  // L in the lower triangle; its inverse X, transposed, in the upper one
-  // (X(r, c) at A[r*PM_LDA + c], r >= c; L's diagonal is kept in rdiag)
-  // (FP32: the FP64 fallback's packed triangle, 2080 doubles, takes the
-  // same 16,640 bytes); all in the caller's LDS buffer of potrf_mw_lds<T>()
+  // (FP32: the FP64 fallback's packed triangle, 2080 doubles, takes A's
+  // 16,640 bytes); all in the caller's LDS buffer of potrf_mw_lds<T>()
   T* const A = reinterpret_cast<T*>(smem);
   T* const rdiag = A + 64 * PM_LDA;
   T* const dg = rdiag + 64;
@@ -580,74 +778,78 @@ __device__ __forceinline__ void potrf_mw_block(const FrontDesc* __restrict__ fr,
   __builtin_amdgcn_s_setprio(3);  // the panel chain is the critical path
   const FrontDesc d = fr[t.front];
   const long long m = d.m;
-  const int kb = t.kb, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int kb = t.kb, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   T* const gp = L + d.offL + t.k0 + (long long)t.k0 * m;
-  // the lower triangle (identity padding beyond kb, zeros above), the 16
-  // loads of a thread issued unconditionally and in flight together (an
-  // entry outside the triangle reads the block's first entry and drops it)
-  T v[16];
+  if constexpr (!STAGED) {
+    // the 16 loads of a thread issued unconditionally and in flight together
+    // (an entry outside the triangle reads the block's first entry and drops it)
+    T v[16];
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int c = wave + 4 * q;
-    const bool ok = lane < kb && c < kb && lane >= c;
-    v[q] = *(ok ? gp + lane + c * m : gp);
-  }
+    for (int q = 0; q < 16; q++) {
+      const int c = wave + 4 * q;
+      v[q] = *(lane < kb && c < kb && lane >= c ? gp + lane + c * m : gp);
+    }
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int c = wave + 4 * q;
-    if (!(lane < kb && c < kb && lane >= c)) v[q] = lane == c ? (T)1 : (T)0;
-    A[c * PM_LDA + lane] = v[q];
-    if (lane == c) dg[c] = v[q];
+    for (int q = 0; q < 16; q++) pm_stage<T>(A, dg, lane, wave + 4 * q, kb, v[q]);
   }
   if (tid == 0) flagged = 0;
   __syncthreads();
   bool bad = false, grow = false;
-#pragma clang loop unroll(full)
-  for (int p = 0; p < 4; p++) {
+  // columns 16 b .. 16 b + 15 of L to the panel, by the nw waves from w0 on
+  auto store_L = [&](int b, int w0, int nw) {
+    for (int c = 16 * b + wave - w0; c < 16 * b + 16; c += nw)
+      if (lane < kb && c < kb && lane >= c) gp[lane + c * m] = A[c * PM_LDA + lane];
+  };
+  // rows r0 .. r1-1 of the inverse, row-major, X(i, j) at Inv[i*64 + j] (zero
+  // outside the block's kb x kb), likewise
+  T* const iv = Inv + d.offI + (long long)(t.k0 / 64) * 4096;
+  auto store_X = [&](int r0, int r1, int w0, int nw) {
+    for (int i = r0 + wave - w0; i < r1; i += nw) {
+      const T x = i == lane ? rdiag[i] : A[i * PM_LDA + lane];
+      iv[i * 64 + lane] = (i < kb && lane < kb && i >= lane) ? x : (T)0;
+    }
+  };
+  // the panels that hold columns of the block; beyond them A is the identity
+  const int last = (kb - 1) >> 4;
+  acc_t S;  // waves 1-3: the sum of X's block (last, j), j = inv_j
+  int inv_j = -1;
+  for (int p = 0; p <= last; p++) {
+    const bool mid = p >= 2;
     if (wave == 0) {
-      const int c0 = 16 * p;
-      T r[16];
-#pragma unroll
-      for (int c = 0; c < 16; c++) r[c] = A[(c0 + c) * PM_LDA + lane];
-      T myrd = (T)1;
-#pragma clang loop unroll(full)
-      for (int q = 0; q < 16; q++) {
-        const int k = c0 + q;
-        T pv = rlane(r[q], k);
-        if constexpr (sizeof(T) == 4) {
-          if (pv < (T)GROW_TAU * dg[k]) grow = true;
-        }
-        // a nonpositive pivot is recorded beside the chain; its NaNs or
-        // infinities run on through a factor that is reported as failed
-        bad = bad || !(pv > (T)0);
-        T dk, rdk;
-        sqrt_pair(pv, dk, rdk);
-        const T lik = r[q] * rdk;
-        r[q] = lane == k ? dk : lik;
-        myrd = lane == k ? rdk : myrd;
-        // (no register barrier: 16 columns cannot spill, and the scheduler
-        // can then overlap the next pivot's chain with these updates)
-#pragma clang loop unroll(full)
-        for (int j = q + 1; j < 16; j++) r[j] -= lik * rlane(lik, c0 + j);
+      if (p < last) pm_panel<T, true>(A, rdiag, dg, p, lane, mid, bad, grow);
+      else pm_panel<T, false>(A, rdiag, dg, p, lane, mid, bad, grow);
+    } else if (p > 0) {
+      // row i of the inverse (wave 1: X_ii; waves 2 and 3: the blocks j = 0
+      // and 1, their sums first) and the updates by panel i that the panel
+      // now factored does not wait for
+      const int i = p - 1, j = wave == 1 ? i : wave - 2;
+      int n = 0;
+      for (int R = p + 1; R <= last; R++)
+        for (int Q = R; Q <= last; Q++)
+          if (1 + n++ % 3 == wave) pm_block_update<T>(A, Q, R, i, lane);
+      if (wave == 1) pm_inv_diag<T>(A, rdiag, Ts[wave], i, lane);
+      // (FP32 keeps the input in the panel, for the fallback, until the end)
+      else if (sizeof(T) == 8) store_L(i, 2, 2);
+      acc_t Sij;
+      if (wave > 1 && j < i) Sij = pm_inv_sum<T>(A, rdiag, i, j, lane);
+      if (mid) __syncthreads();  // X_ii
+      if (wave > 1 && j < i) pm_inv_block<T>(A, rdiag, Ts[wave], i, j, Sij, lane);
+      // before the last panel: the sums of its row of X, each from blocks
+      // that other panels' times completed and the wave's own
+      if (p == last && j <= i && (wave == 1 || j < i)) {
+        if (wave == 1) wave_lds_fence();
+        S = pm_inv_sum<T>(A, rdiag, last, j, lane);
+        inv_j = j;
       }
-#pragma unroll
-      for (int c = 0; c < 16; c++) A[(c0 + c) * PM_LDA + lane] = lane >= c0 + c ? r[c] : (T)0;
-      if (lane >= c0 && lane < c0 + 16) rdiag[lane] = myrd;
     }
     __syncthreads();
-    if (p < 3) {
-      // the blocks (Q, R), Q >= R > p, round robin over the waves
-      int n = 0;
-#pragma clang loop unroll(full)
-      for (int R = p + 1; R < 4; R++)
-#pragma clang loop unroll(full)
-        for (int Q = R; Q < 4; Q++) {
-          if ((n & 3) == wave) pm_block_update<T>(A, Q, R, p, lane);
-          n++;
-        }
+    if (p < last) {  // the next panel's blocks
+      if (wave < last - p) pm_block_update<T>(A, p + 1 + wave, p + 1, p, lane);
       __syncthreads();
     }
   }
+  bool whole_inverse = false;
   if constexpr (sizeof(T) == 4) {
     // a flagged block (nonpositive pivot or pivot growth) again in FP64 from
     // its input, by wave 0 in the packed triangle
@@ -662,93 +864,48 @@ __device__ __forceinline__ void potrf_mw_block(const FrontDesc* __restrict__ fr,
         bool bad64 = false;
         wave_chol_packed_f64(P, lane, ~0ULL, bad64);
         T rd = (T)(1.0 / P[ptri(lane, lane)]);
-        T v[64];
+        T w[64];
 #pragma unroll
-        for (int c = 0; c < 64; c++) v[c] = c <= lane ? (T)P[ptri(lane, c)] : (T)0;
+        for (int c = 0; c < 64; c++) w[c] = c <= lane ? (T)P[ptri(lane, c)] : (T)0;
         wave_lds_fence();
 #pragma unroll
-        for (int c = 0; c < 64; c++) A[c * PM_LDA + lane] = v[c];
+        for (int c = 0; c < 64; c++) A[c * PM_LDA + lane] = w[c];
         rdiag[lane] = rd;
         bad = bad64;
         if (lane == 0) atomicAdd(info + 1, 1);
       }
       __syncthreads();
+      whole_inverse = true;
     }
   }
   if (tid == 0 && bad) atomicOr(info, 1);
-  // L back to the panel
-#pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int c = wave + 4 * q;
-    if (lane < kb && c < kb && lane >= c) gp[lane + c * m] = A[c * PM_LDA + lane];
-  }
-  __syncthreads();  // the diagonal of A is overwritten by X's next
-  // inverse: the diagonal 16 x 16 blocks, lane (b, c16) holds column c16 of X_bb
-  const int c16 = lane & 15, g = lane >> 4;
-  if (wave == 0) {
-    const int b = g;
-    T x[16];
-#pragma clang loop unroll(full)
-    for (int i = 0; i < 16; i++) {
-      asm volatile("" ::: "memory");  // one row's entries in registers at a time
-      T a0 = (i == c16) ? (T)1 : (T)0, a1 = (T)0;
-#pragma clang loop unroll(full)
-      for (int tt = 0; tt < i; tt += 2) {
-        a0 -= A[(16 * b + tt) * PM_LDA + 16 * b + i] * x[tt];
-        if (tt + 1 < i) a1 -= A[(16 * b + tt + 1) * PM_LDA + 16 * b + i] * x[tt + 1];
+  if (whole_inverse) {
+    // X from the new factor: the diagonal blocks, then by distance
+    pm_inv_diag<T>(A, rdiag, Ts[wave], wave, lane);
+    __syncthreads();
+    for (int dd = 1; dd < 4; dd++) {
+      const int i = wave + dd;
+      if (i < 4) {
+        const acc_t s = pm_inv_sum<T>(A, rdiag, i, wave, lane);
+        pm_inv_block<T>(A, rdiag, Ts[wave], i, wave, s, lane);
       }
-      x[i] = (a0 + a1) * rdiag[16 * b + i];
-      asm volatile("" : "+v"(x[i]));
+      __syncthreads();
     }
-    wave_lds_fence();  // every row of L_bb read before X_bb takes the upper triangle
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-      if (i >= c16) A[(16 * b + i) * PM_LDA + 16 * b + c16] = x[i];
+    for (int b = 0; b < 4; b++) store_L(b, 0, 4);
+    store_X(0, 64, 0, 4);
+    return;
+  }
+  // X's last row of blocks, and beside its diagonal block what is complete
+  if (wave == 0) {
+    pm_inv_diag<T>(A, rdiag, Ts[wave], last, lane);
+  } else {
+    for (int b = sizeof(T) == 8 ? last : 0; b <= last; b++) store_L(b, 1, 3);
+    store_X(0, 16 * last, 1, 3);
   }
   __syncthreads();
-  // off-diagonal blocks by distance: X_ij = -X_ii (sum_{k=j}^{i-1} L_ik X_kj);
-  // X_kj's entries above its diagonal (k = j) and X_ii's are masked: there
-  // the upper triangle holds L
-#pragma clang loop unroll(full)
-  for (int dd = 1; dd < 4; dd++) {
-    const int j = wave, i = wave + dd;
-    if (i < 4) {
-      acc_t acc;
-#pragma clang loop unroll(full)
-      for (int e = 0; e < 4; e++) acc[e] = (T)0;
-      for (int k = j; k < i; k++)
-#pragma clang loop unroll(full)
-        for (int st = 0; st < 4; st++) {
-          const int kr = 4 * st + g;
-          const T a = A[(16 * k + kr) * PM_LDA + 16 * i + c16];
-          const T bv = (k > j || kr >= c16) ? A[(16 * k + kr) * PM_LDA + 16 * j + c16] : (T)0;
-          acc = Mfma<T>::step(a, bv, acc);
-        }
-      T* ts = Ts[wave];
-#pragma clang loop unroll(full)
-      for (int e = 0; e < 4; e++) ts[Mfma<T>::drow(lane, e) * 17 + c16] = acc[e];
-      wave_lds_fence();
-      acc_t xr;
-#pragma clang loop unroll(full)
-      for (int e = 0; e < 4; e++) xr[e] = (T)0;
-#pragma clang loop unroll(full)
-      for (int st = 0; st < 4; st++) {
-        const int kr = 4 * st + g;
-        const T a = c16 >= kr ? A[(16 * i + c16) * PM_LDA + 16 * i + kr] : (T)0;
-        xr = Mfma<T>::step(a, ts[kr * 17 + c16], xr);
-      }
-#pragma clang loop unroll(full)
-      for (int e = 0; e < 4; e++) A[(16 * i + Mfma<T>::drow(lane, e)) * PM_LDA + 16 * j + c16] = -xr[e];
-    }
-    __syncthreads();
-  }
-  // Inv row-major, X(i, j) at Inv[i*64 + j] (zero outside the block's kb x kb)
-  T* const iv = Inv + d.offI + (long long)(t.k0 / 64) * 4096;
-#pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int idx = tid + 256 * q, i = idx >> 6, j = idx & 63;
-    iv[idx] = (i < kb && j < kb && i >= j) ? A[i * PM_LDA + j] : (T)0;
-  }
+  if (inv_j >= 0) pm_inv_block<T>(A, rdiag, Ts[wave], last, inv_j, S, lane);
+  __syncthreads();
+  store_X(16 * last, 64, 0, 4);
 }
 
 template <typename T>
@@ -758,7 +915,7 @@ __global__ __launch_bounds__(256) void k_potrf_mw(const FrontDesc* __restrict__ 
                                                   int* __restrict__ info, int fallback)
 {
   __shared__ __align__(16) unsigned char smem[potrf_mw_lds<T>()];
-  potrf_mw_block<T>(fr, tasks[blockIdx.x], L, Inv, info, fallback, smem);
+  potrf_mw_block<T, false>(fr, tasks[blockIdx.x], L, Inv, info, fallback, smem);
 }
 
 // Whole front with m <= 64 in one wavefront: lane i holds row i of the
@@ -1889,6 +2046,10 @@ __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict
     __syncthreads();
     mma_half(acc, As, As);
   }
+  const bool pf = t.pf_front >= 0;
+  T* const PA = reinterpret_cast<T*>(smem);
+  T* const pdg = PA + 64 * PM_LDA + 64;
+  if (pf) __syncthreads();  // As is read before the block takes its place
 #pragma unroll
   for (int a = 0; a < 2; a++)
 #pragma unroll
@@ -1896,11 +2057,13 @@ __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int i = wr + 16 * a + c16, j = wc + 16 * b + Mfma<T>::drow(lane, r);
-        if (i < t.Md && j < t.Md && i >= j) L[t.d_off + i + j * ld] = dv[a][b][r] - acc[a][b][r];
+        const T v = dv[a][b][r] - acc[a][b][r];
+        if (pf) pm_stage<T>(PA, pdg, i, j, t.Md, v);
+        if ((!pf || sizeof(T) == 4) && i < t.Md && j < t.Md && i >= j) L[t.d_off + i + j * ld] = v;
       }
-  if (t.pf_front < 0) return;
-  __syncthreads();  // the block's update is stored, and As read, before the POTRF
-  potrf_mw_block<T>(fr, PanelTask{t.pf_front, t.pf_k0, t.Md, 0, 0}, L, Inv, info, fallback, smem);
+  if (!pf) return;
+  // (its barrier after the prologue: the block is staged, and in FP32 stored)
+  potrf_mw_block<T, true>(fr, PanelTask{t.pf_front, t.pf_k0, t.Md, 0, 0}, L, Inv, info, fallback, smem);
 }
 
 // 128 x 128 tile for the large trailing updates and SYRKs: 4 waves (2 x 2),
