@@ -1252,10 +1252,10 @@ struct Emitter {
     if (E.kernel(__VA_ARGS__) != 0) return -1; \
   } while (0)
 
-// LDS per CU is 160 KiB.  Side-lane tiles: FP64 two per CU (waves of 104
-// registers, leaving 304 on each SIMD for the 288-register POTRF wave and
-// 48 KiB of LDS for its 37 KiB); FP32 four per CU (64-register waves, POTRF
-// 152 registers and 18.5 KiB).
+// LDS per CU is 160 KiB.  Side-lane 64-tiles: FP64 two per CU (waves of 104
+// registers, leaving 304 on each SIMD and 52 KiB of LDS for a panel step's
+// workgroup: waves of 253 registers, 51 KiB); FP32 four per CU (64-register
+// waves, the panel step's 153 registers and 26 KiB).
 template <typename T> constexpr int SIDE_WGS = sizeof(T) == 8 ? 2 : 4;
 #define SIDE_PAD_MAX_TILES_FP64 4096
 #ifndef LAT_TILES_MAX
@@ -1265,7 +1265,7 @@ template <typename T>
 static unsigned side_lds_pad()
 {
   const unsigned tile_lds = 2u * 64 * (16 + 2) * sizeof(T);  // As + Bs of the 64x64 tile
-  const unsigned per_wg = (160u * 1024 - (sizeof(T) == 8 ? 48u : 24u) * 1024) / SIDE_WGS<T>;
+  const unsigned per_wg = (160u * 1024 - (sizeof(T) == 8 ? 52u : 27u) * 1024) / SIDE_WGS<T>;
   return per_wg > tile_lds ? per_wg - tile_lds : 0;
 }
 

@@ -518,18 +518,20 @@ __global__ __launch_bounds__(64) void k_potrf_wave(const FrontDesc* __restrict__
 // The diagonal block of a panel step by four waves (256 threads), in LDS
 // (column-major, A(i, c) at A[c*PM_LDA + i]).  What bounds it is latency: the
 // chain of 64 pivots (broadcast, reciprocal square root, scaling, the column's
-// updates: 190 to 260 cycles each), then the inverse.  So wave 0 runs
-// the chain alone, in 16-column panels (pm_panel), and the other waves do
-// everything else beside it: the updates of the blocks that the next panel
-// does not touch, and the rows of the inverse X = L^{-1} as far as L is
-// known.  Only the next panel's blocks are updated between two panels
-// (rank-16 MFMA updates, one block per wave), and after the last panel only
-// its own block of X and one product per block of X's last row are left.
+// updates, some 25 instructions at 6 cycles each from a single wave).  So the
+// chain runs in 16-column panels, whose diagonal block two waves factor, each
+// for itself: wave 0 solves the rows below with it, wave 1 inverts it.  The
+// other two waves do beside them what needs earlier panels only: the updates
+// of the blocks that the next panel does not touch, the blocks of the inverse
+// X = L^{-1} left of its diagonal, and L's way back to memory.  Between two
+// panels only the next one's blocks are updated (rank-16 MFMA updates, one
+// block per wave), and after the last panel only one product per block of X's
+// last row is left.
 // L stays in the lower triangle; X, transposed, in the strict upper one
 // (X(r, c) at A[r*PM_LDA + c], r > c), its diagonal is rdiag.
-// Measured on one block, 64 columns, launch included: FP64 18.3 -> 13.7 us,
-// FP32 18.3 -> 15.9 us, against panels whose multipliers all came by readlane
-// and an inverse after the last panel.
+// Measured on one block, 64 columns, launch included: FP64 18.3 -> 11.9 us,
+// FP32 18.3 -> 15.3 us, against panels by one wave whose multipliers came by
+// readlane, and an inverse after the last panel.
 // The MFMA steps apply their products as one fused multiply-add after another
 // in k order, so L and the inverse are bitwise those of k_potrf_wave.
 #define PM_LDA 65
@@ -615,61 +617,110 @@ __device__ __forceinline__ void static_for(F&& f)
   }
 }
 
-// Panel p (columns 16p .. 16p+15) by one wave.  Every 16 lanes hold a copy of
-// the panel's diagonal block (lane li its row li), and with SUB each lane also
-// the row `lane` of the whole panel: the pivot and a column's multipliers are
-// then operands broadcast within the 16 lanes, and nothing of a step waits
-// for a scalar register (27 cycles after a readlane) or for LDS.  A dependent
-// FP64 operation takes 5 cycles, so the panel is bound by the instructions it
-// issues (about 6 cycles apiece from a single wave).  The pivots are collected, one a lane; the diagonal, its reciprocals
-// and the checks follow for all 16 at once.  Nothing reads the entries above
-// the diagonal, which hold no defined values.  `mid`: the barrier halfway, at
-// which the other waves hand over within this panel's time.  (A nonpositive
-// pivot's NaNs or infinities run on through a factor that is reported as
-// failed.)
-template <typename T, bool SUB>
-__device__ __forceinline__ void pm_panel(T* A, T* rdiag, const T* dg, int p, int lane, bool mid,
-                                         bool& bad, bool& grow)
+// One step of a panel: column q of the diagonal block, of which every 16 lanes
+// hold a copy (lane li its row li in r).  The pivot and the column's multipliers
+// are operands broadcast within the 16 lanes, so nothing of a step waits for a
+// scalar register (27 cycles after a readlane) or for LDS.  The entries above
+// the diagonal hold no defined values, and nothing reads them.
+template <int q, typename T>
+__device__ __forceinline__ T pm_column(T (&r)[16], T& rdk)
+{
+  const T pv = bcast16<q>(r[q]);
+  T dk;
+  if constexpr (sizeof(T) == 8) rdk = rsqrt_step(pv, __builtin_amdgcn_rsq(pv));
+  else sqrt_pair(pv, dk, rdk);
+  const T l = r[q] * rdk;
+  if constexpr (q < 15) {
+    fms_bcast16_first<q + 1>(r[q + 1], l, l);
+    static_for<q + 2, 16>([&](auto J) { fms_bcast16<J>(r[J], l, l, r[q + 1]); });
+  }
+  return l;
+}
+
+// Panel p's rows below its diagonal block (columns 16p .. 16p+15) by one wave,
+// lane = row.  The diagonal block is another wave's to write (pm_panel_diag),
+// which reads it at the same time.
+template <typename T>
+__device__ __forceinline__ void pm_panel_rows(T* A, int p, int lane)
 {
   const int c0 = 16 * p, li = lane & 15;
   T* const Ac = A + c0 * PM_LDA;
-  T r[16], rs[16], P = (T)1;
+  T r[16], rs[16];
 #pragma unroll
   for (int c = 0; c < 16; c++) {
     r[c] = Ac[c * PM_LDA + c0 + li];
-    if (SUB) rs[c] = Ac[c * PM_LDA + lane];
+    rs[c] = Ac[c * PM_LDA + lane];
   }
   static_for<0, 16>([&](auto Q) {
     constexpr int q = Q;
-    if (q == 8 && mid) __syncthreads();
-    P = li == q ? r[q] : P;
-    const T pv = bcast16<q>(r[q]);
-    T dk, rdk;
-    if constexpr (sizeof(T) == 8) rdk = rsqrt_step(pv, __builtin_amdgcn_rsq(pv));
-    else sqrt_pair(pv, dk, rdk);
-    const T l = r[q] * rdk;
-    const T ls = SUB ? rs[q] * rdk : l;
-    if constexpr (q < 15) {
-      fms_bcast16_first<q + 1>(r[q + 1], l, l);
-      static_for<q + 2, 16>([&](auto J) { fms_bcast16<J>(r[J], l, l, r[q + 1]); });
-      if (SUB) static_for<q + 1, 16>([&](auto J) { fms_bcast16<J>(rs[J], l, ls, r[q + 1]); });
-    }
-    Ac[q * PM_LDA + (SUB ? lane : c0 + li)] = ls;
+    T rdk;
+    const T l = pm_column<q>(r, rdk);
+    rs[q] = rs[q] * rdk;
+    if constexpr (q < 15)
+      static_for<q + 1, 16>([&](auto J) { fms_bcast16<J>(rs[J], l, rs[q], r[q + 1]); });
   });
-  T d, rd;
-  sqrt_pair(P, d, rd);
-  if (lane < 16) {
-    rdiag[c0 + li] = rd;
-    Ac[li * PM_LDA + c0 + li] = d;
+  if (lane >= c0 + 16) {
+#pragma unroll
+    for (int c = 0; c < 16; c++) Ac[c * PM_LDA + lane] = rs[c];
   }
+}
+
+// Panel p's diagonal block and its inverse by one wave.  X_pp = L_pp^{-1}, lane
+// li holding column li: x_i = (delta_ic - sum_t l_it x_t) / l_ii, the even and
+// the odd t summed apart, column q as soon as it exists.  The pivots are
+// collected, one a lane; the diagonal, its reciprocals and the checks follow
+// for all 16 at once.  (A nonpositive pivot's NaNs or infinities run on through
+// a factor that is reported as failed.)  r holds the block's columns, d its
+// diagonal and x the inverse: the caller stores them (pm_diag_store) once the
+// wave of the rows below has read the block.
+template <typename T>
+__device__ __forceinline__ void pm_panel_diag(const T* A, T* rdiag, const T* dg, int p, int lane,
+                                              T (&r)[16], T& d, T (&x)[16], bool& bad, bool& grow)
+{
+  const int c0 = 16 * p, li = lane & 15;
+  const T* const Ac = A + c0 * PM_LDA + c0 + li;
+  T s[2][16], P = (T)1;
+#pragma unroll
+  for (int c = 0; c < 16; c++) {
+    r[c] = Ac[c * PM_LDA];
+    s[0][c] = c == li ? (T)1 : (T)0;
+    s[1][c] = (T)0;
+  }
+  static_for<0, 16>([&](auto Q) {
+    constexpr int q = Q;
+    P = li == q ? r[q] : P;
+    T rdk;
+    const T l = pm_column<q>(r, rdk);
+    x[q] = (s[0][q] + s[1][q]) * rdk;
+    if constexpr (q < 15)
+      static_for<q + 1, 16>([&](auto J) { fms_bcast16<J>(s[q & 1][J], l, x[q], r[q + 1]); });
+    r[q] = l;
+  });
+  T rd;
+  sqrt_pair(P, d, rd);
+  if (lane < 16) rdiag[c0 + li] = rd;
   bad = bad || __ballot(!(P > (T)0)) != 0;
   if constexpr (sizeof(T) == 4) grow = grow || __ballot(P < (T)GROW_TAU * dg[c0 + li]) != 0;
 }
 
-// X_bb = L_bb^{-1} of a 16 x 16 diagonal block by one wave, lane c16 holding
-// column c16: x_i = (delta_ic - sum_t l_it x_t) / l_ii, the even and the odd t
-// summed apart; column by column, so that x_t waits only for x_{t-1}, with
-// column t of L one entry a lane and its entries broadcast.  The entries below
+// The diagonal block and its inverse into A: the columns whole (above the
+// diagonal they hold nothing), the diagonal, then the inverse above it, a lane
+// without an entry of the inverse's column storing into `dump` (16 values)
+template <typename T>
+__device__ __forceinline__ void pm_diag_store(T* A, T* dump, int p, int lane, const T (&r)[16], T d,
+                                              const T (&x)[16])
+{
+  const int li = lane & 15;
+  T* const to = A + (16 * p) * PM_LDA + 16 * p + li;
+#pragma unroll
+  for (int c = 0; c < 16; c++) to[c * PM_LDA] = r[c];
+  to[li * PM_LDA] = d;
+#pragma unroll
+  for (int i = 1; i < 16; i++) *(i > li ? to + i * PM_LDA : dump + li) = x[i];
+}
+
+// X_bb = L_bb^{-1} from L in A, as pm_panel_diag forms it beside the factor (for
+// the FP64 fallback's factor), column t of L one entry a lane.  The entries below
 // the diagonal go to the transposed position; a lane without one stores into
 // `dump` (16 values)
 template <typename T>
@@ -720,14 +771,18 @@ __device__ __forceinline__ typename Mfma<T>::acc_t pm_inv_sum(const T* A, const 
   return acc;
 }
 
-// X_ij = -X_ii S_ij by one wave (ts: its 16 x 17 staging tile)
+// X_ij = -X_ii S_ij by one wave, S_ij staged in a 16 x 17 tile first (by
+// pm_inv_stage, in the same wave or before a barrier)
 template <typename T>
-__device__ __forceinline__ void pm_inv_block(T* A, const T* rdiag, T* ts, int i, int j,
-                                             const typename Mfma<T>::acc_t& S, int lane)
+__device__ __forceinline__ void pm_inv_stage(T* ts, const typename Mfma<T>::acc_t& S, int lane)
+{
+#pragma clang loop unroll(full)
+  for (int e = 0; e < 4; e++) ts[Mfma<T>::drow(lane, e) * 17 + (lane & 15)] = S[e];
+}
+template <typename T>
+__device__ __forceinline__ void pm_inv_block(T* A, const T* rdiag, const T* ts, int i, int j, int lane)
 {
   const int c16 = lane & 15, g = lane >> 4;
-#pragma clang loop unroll(full)
-  for (int e = 0; e < 4; e++) ts[Mfma<T>::drow(lane, e) * 17 + c16] = S[e];
   wave_lds_fence();
   typename Mfma<T>::acc_t xr;
 #pragma clang loop unroll(full)
@@ -750,13 +805,13 @@ template <typename T>
 constexpr int potrf_mw_lds() { return (int)sizeof(T) * (64 * PM_LDA + 64 + 64 + 4 * 16 * 17) + 16; }
 
 // entry (i, j) of the block as potrf_mw_block wants it in LDS: the lower
-// triangle of its kb x kb, the identity beyond
+// triangle of its kb x kb (above it anything), the identity beyond
 template <typename T>
 __device__ __forceinline__ void pm_stage(T* A, T* dg, int i, int j, int kb, T v)
 {
-  if (!(i < kb && j < kb && i >= j)) v = i == j ? (T)1 : (T)0;
+  if (kb < 64 && !(i < kb && j < kb)) v = i == j ? (T)1 : (T)0;
   A[j * PM_LDA + i] = v;
-  if (i == j) dg[i] = v;
+  if (sizeof(T) == 4 && i == j) dg[i] = v;
 }
 
 // STAGED: the caller has put the block into A and dg (pm_stage), and has
@@ -796,67 +851,82 @@ __device__ __forceinline__ void potrf_mw_block(const FrontDesc* __restrict__ fr,
   if (tid == 0) flagged = 0;
   __syncthreads();
   bool bad = false, grow = false;
-  // columns 16 b .. 16 b + 15 of L to the panel, by the nw waves from w0 on
-  auto store_L = [&](int b, int w0, int nw) {
-    for (int c = 16 * b + wave - w0; c < 16 * b + 16; c += nw)
-      if (lane < kb && c < kb && lane >= c) gp[lane + c * m] = A[c * PM_LDA + lane];
+  // four columns of L (c, c + dc, ..) to the panel, and four rows of the
+  // inverse, row-major, X(i, j) at Inv[i*64 + j] (zero outside the block's
+  // kb x kb): by one wave, the LDS reads in flight together
+  auto store_L = [&](int c, int dc) {
+    T w[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = A[(c + dc * e) * PM_LDA + lane];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (lane < kb && c + dc * e < kb && lane >= c + dc * e) gp[lane + (c + dc * e) * m] = w[e];
   };
-  // rows r0 .. r1-1 of the inverse, row-major, X(i, j) at Inv[i*64 + j] (zero
-  // outside the block's kb x kb), likewise
   T* const iv = Inv + d.offI + (long long)(t.k0 / 64) * 4096;
-  auto store_X = [&](int r0, int r1, int w0, int nw) {
-    for (int i = r0 + wave - w0; i < r1; i += nw) {
-      const T x = i == lane ? rdiag[i] : A[i * PM_LDA + lane];
-      iv[i * 64 + lane] = (i < kb && lane < kb && i >= lane) ? x : (T)0;
+  auto store_X = [&](int i, int di) {
+    T w[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = i + di * e;
+      w[e] = *(r == lane ? rdiag + r : A + r * PM_LDA + lane);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = i + di * e;
+      iv[r * 64 + lane] = (r < kb && lane < kb && r >= lane) ? w[e] : (T)0;
     }
   };
   // the panels that hold columns of the block; beyond them A is the identity
   const int last = (kb - 1) >> 4;
-  acc_t S;  // waves 1-3: the sum of X's block (last, j), j = inv_j
-  int inv_j = -1;
+  acc_t S;  // waves 2 and 3: the sum of X's next block of column j
+  const int j = wave - 2;
   for (int p = 0; p <= last; p++) {
-    const bool mid = p >= 2;
+    T r[16], d, x[16];  // wave 1
     if (wave == 0) {
-      if (p < last) pm_panel<T, true>(A, rdiag, dg, p, lane, mid, bad, grow);
-      else pm_panel<T, false>(A, rdiag, dg, p, lane, mid, bad, grow);
+      // (in the last panel's time, which has no rows for it: the rows of X that
+      // are complete; FP32 keeps to the end, for the fallback)
+      if (p < last) pm_panel_rows<T>(A, p, lane);
+      else if (sizeof(T) == 8)
+        for (int r = 0; r < 16 * (last - 1); r += 4) store_X(r, 1);
+    } else if (wave == 1) {
+      pm_panel_diag<T>(A, rdiag, dg, p, lane, r, d, x, bad, grow);
+      if (p == last) pm_diag_store<T>(A, Ts[0], p, lane, r, d, x);
     } else if (p > 0) {
-      // row i of the inverse (wave 1: X_ii; waves 2 and 3: the blocks j = 0
-      // and 1, their sums first) and the updates by panel i that the panel
-      // now factored does not wait for
-      const int i = p - 1, j = wave == 1 ? i : wave - 2;
+      // the updates by panel i that this panel does not wait for
+      const int i = p - 1;
       int n = 0;
       for (int R = p + 1; R <= last; R++)
         for (int Q = R; Q <= last; Q++)
-          if (1 + n++ % 3 == wave) pm_block_update<T>(A, Q, R, i, lane);
-      if (wave == 1) pm_inv_diag<T>(A, rdiag, Ts[wave], i, lane);
-      // (FP32 keeps the input in the panel, for the fallback, until the end)
-      else if (sizeof(T) == 8) store_L(i, 2, 2);
-      acc_t Sij;
-      if (wave > 1 && j < i) Sij = pm_inv_sum<T>(A, rdiag, i, j, lane);
-      if (mid) __syncthreads();  // X_ii
-      if (wave > 1 && j < i) pm_inv_block<T>(A, rdiag, Ts[wave], i, j, Sij, lane);
-      // before the last panel: the sums of its row of X, each from blocks
-      // that other panels' times completed and the wave's own
-      if (p == last && j <= i && (wave == 1 || j < i)) {
-        if (wave == 1) wave_lds_fence();
-        S = pm_inv_sum<T>(A, rdiag, last, j, lane);
-        inv_j = j;
+          if (3 - (n++ & 1) == wave) pm_block_update<T>(A, Q, R, i, lane);
+      // X's block (i, j) and the sum of its block (p, j); wave 3 also the sum
+      // of block (3, 2), which wave 1 takes from its tile
+      if (j < i) {
+        pm_inv_stage<T>(Ts[wave], S, lane);
+        pm_inv_block<T>(A, rdiag, Ts[wave], i, j, lane);
       }
+      if (j < p) S = pm_inv_sum<T>(A, rdiag, p, j, lane);
+      if (p == 3 && wave == 3) pm_inv_stage<T>(Ts[1], pm_inv_sum<T>(A, rdiag, 3, 2, lane), lane);
+      // (FP32 keeps the input in the panel, for the fallback, until the end)
+      if (sizeof(T) == 8)
+        for (int c = 0; c < 2; c++) store_L(16 * i + 4 * (wave - 2) + c * 8, 1);
     }
     __syncthreads();
-    if (p < last) {  // the next panel's blocks
-      if (wave < last - p) pm_block_update<T>(A, p + 1 + wave, p + 1, p, lane);
+    if (p < last) {
+      if (wave == 1) pm_diag_store<T>(A, Ts[0], p, lane, r, d, x);
+      // the next panel's blocks, by the other waves
+      else if (p + 1 + (wave > 0 ? wave - 1 : 0) <= last)
+        pm_block_update<T>(A, p + 1 + (wave > 0 ? wave - 1 : 0), p + 1, p, lane);
       __syncthreads();
     }
   }
   bool whole_inverse = false;
   if constexpr (sizeof(T) == 4) {
     // a flagged block (nonpositive pivot or pivot growth) again in FP64 from
-    // its input, by wave 0 in the packed triangle
-    if (wave == 0 && fallback && (bad || grow) && lane == 0) flagged = 1;
+    // its input, by wave 1 in the packed triangle
+    if (wave == 1 && fallback && (bad || grow) && lane == 0) flagged = 1;
     __syncthreads();
     if (flagged) {
-      if (wave == 0) {
+      if (wave == 1) {
         static_assert(sizeof(T) != 4 || 64 * PM_LDA * sizeof(T) >= 2080 * sizeof(double), "");
         double* P = reinterpret_cast<double*>(A);  // the FP32 factor is discarded
         for (int c = 0; c <= lane; c++)
@@ -878,34 +948,41 @@ __device__ __forceinline__ void potrf_mw_block(const FrontDesc* __restrict__ fr,
       whole_inverse = true;
     }
   }
-  if (tid == 0 && bad) atomicOr(info, 1);
-  if (whole_inverse) {
-    // X from the new factor: the diagonal blocks, then by distance
-    pm_inv_diag<T>(A, rdiag, Ts[wave], wave, lane);
-    __syncthreads();
-    for (int dd = 1; dd < 4; dd++) {
-      const int i = wave + dd;
-      if (i < 4) {
-        const acc_t s = pm_inv_sum<T>(A, rdiag, i, wave, lane);
-        pm_inv_block<T>(A, rdiag, Ts[wave], i, wave, s, lane);
-      }
+  if (tid == 64 && bad) atomicOr(info, 1);
+  if constexpr (sizeof(T) == 4) {
+    if (whole_inverse) {
+      // X from the new factor: the diagonal blocks, then by distance
+      pm_inv_diag<T>(A, rdiag, Ts[wave], wave, lane);
       __syncthreads();
+      for (int dd = 1; dd < 4; dd++) {
+        const int i = wave + dd;
+        if (i < 4) {
+          pm_inv_stage<T>(Ts[wave], pm_inv_sum<T>(A, rdiag, i, wave, lane), lane);
+          pm_inv_block<T>(A, rdiag, Ts[wave], i, wave, lane);
+        }
+        __syncthreads();
+      }
+      for (int b = 0; b < 4; b++) {
+        store_L(16 * b + wave, 4);
+        store_X(16 * b + wave, 4);
+      }
+      return;
     }
-    for (int b = 0; b < 4; b++) store_L(b, 0, 4);
-    store_X(0, 64, 0, 4);
-    return;
   }
-  // X's last row of blocks, and beside its diagonal block what is complete
+  // X's last row of blocks, and beside it what is complete
   if (wave == 0) {
-    pm_inv_diag<T>(A, rdiag, Ts[wave], last, lane);
-  } else {
-    for (int b = sizeof(T) == 8 ? last : 0; b <= last; b++) store_L(b, 1, 3);
-    store_X(0, 16 * last, 1, 3);
+    if (sizeof(T) == 8)
+      for (int c = 0; c < 4; c++) store_L(16 * last + 4 * c, 1);
+  } else if (wave == 1) {
+    if (last == 3) pm_inv_block<T>(A, rdiag, Ts[1], 3, 2, lane);
+  } else if (j < last) {
+    pm_inv_stage<T>(Ts[wave], S, lane);
+    pm_inv_block<T>(A, rdiag, Ts[wave], last, j, lane);
   }
   __syncthreads();
-  if (inv_j >= 0) pm_inv_block<T>(A, rdiag, Ts[wave], last, inv_j, S, lane);
-  __syncthreads();
-  store_X(16 * last, 64, 0, 4);
+  if (sizeof(T) == 4)
+    for (int b = 0; b <= last; b++) store_L(16 * b + wave, 4);
+  for (int r = (sizeof(T) == 8 && last > 0 ? 16 * (last - 1) : 0) + 4 * wave; r < 64; r += 16) store_X(r, 1);
 }
 
 template <typename T>
@@ -1855,135 +1932,171 @@ __global__ __launch_bounds__(256) void k_gemm_short(const GemmTask* __restrict__
 //                       complete.
 // The other tiles of the later blocks receive their updates when their own
 // step comes.  The workgroup of the tile that starts the next step's block
-// then factors that block (potrf_mw_block, as k_potrf_mw would in a launch of
-// its own), so an outer panel's steps after the first need one launch each.
-// MFMA layout and 16-deep K chunks as in gemm_tile_short: wave w holds the
-// 32 x 32 sub-tile (wr, wc), element r of acc[a][b] at row wr + 16a + c16 and
-// column wc + 16b + drow(lane, r).
+// then factors that block, handed over in LDS (potrf_mw_block), so an outer
+// panel's steps after the first need one launch each.
+// Most steps have fewer tiles than the GPU has CUs and one wave to a SIMD, so
+// a step lasts as long as its products' slowest wave: 4096 cycles a 64 x 64 x
+// 64 product in FP64 if nothing else comes between the MFMAs.  As in
+// k_gemm_tile128, one operation is issued behind each MFMA: the fragments of
+// the next step, and in the left-looking part the stores of the next 16-deep
+// chunk into the other buffer and the loads of the chunk four ahead (a whole
+// block of columns: an L2 round trip is longer than a chunk).  The inverse is
+// read 16 bytes a lane along its rows and staged as [row][k].  Measured against
+// halves of 32 columns staged and multiplied in turn: one product 7.7K -> 5.6K
+// cycles; POTRF and the four steps of a 256-column outer panel of 2000 rows 113
+// -> 100 us FP64, 106 -> 93 us FP32 (with potrf_mw_block's present form 93, 88).
+// The staging takes 51 KB, so that a workgroup fits beside two of the side
+// lane's.  MFMA layout as in gemm_tile: wave w holds the 32 x 32 sub-tile
+// (wr, wc), element r of acc[a][b] at row wr + 16a + c16 and column
+// wc + 16b + drow(lane, r); k order 16 c + 4 g + step.
 template <typename T>
 __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict__ tasks, T* L,
                                                      T* Inv, const FrontDesc* __restrict__ fr,
                                                      int* __restrict__ info, int fallback)
 {
   typedef typename Mfma<T>::acc_t acc_t;
-  // one LDS buffer: the staging halves As, Bs, then the next block's POTRF
-  constexpr int STAGE = 2 * 2 * 64 * KP * (int)sizeof(T);
+  constexpr int VEC = 16 / (int)sizeof(T);       // rows (or columns) of one load
+  constexpr int RG = 64 / VEC;                   // row groups of a chunk's loads
+  constexpr int NV = 64 * 16 / (VEC * 256);      // loads per operand, chunk and thread
+  constexpr int NI = 64 * 32 / (VEC * 256);      // the same of half the inverse
+  constexpr int LDR = 68, LDK = 32 + VEC;        // [k][row] of the operands, [row][k] of the inverse
+  typedef T vec_t __attribute__((ext_vector_type(VEC)));
+  typedef vec_t vecu_t __attribute__((aligned(sizeof(T))));
+  // left-looking: two 16-deep chunks of A and of B; then all 64 columns of A
+  // and half the inverse; then the next block's POTRF
+  constexpr int STAGE = (64 * LDR + 64 * LDK) * (int)sizeof(T);
+  static_assert(4 * 16 * LDR <= 64 * LDR + 64 * LDK, "");
   __shared__ __align__(16) unsigned char smem[STAGE > potrf_mw_lds<T>() ? STAGE : potrf_mw_lds<T>()];
-  T (*const As)[64][KP] = reinterpret_cast<T (*)[64][KP]>(smem);
-  T (*const Bs)[64][KP] = As + 2;
+  T* const As = reinterpret_cast<T*>(smem);
   __builtin_amdgcn_s_setprio(2);
   const SolveTask t = tasks[blockIdx.x];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   const int c16 = lane & 15, g = lane >> 4;
-  const int li = tid & 63, lk = tid >> 6;  // loader: row li, k = 16 ch + lk + 4q
   const long long ld = t.ld;
-  // issued first: the tile (accumulator layout)
-  acc_t C[2][2];
+  // issued first: the tile (accumulator layout; clamped to the tile, columns
+  // past N become zero when they are staged, rows past M are not stored)
+  acc_t C[2][2], acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; a++)
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = wr + 16 * a + c16, j = wc + 16 * b + Mfma<T>::drow(lane, r);
-        C[a][b][r] = (i < t.M && j < t.N) ? L[t.c_off + i + j * ld] : (T)0;
+        const int i = min(wr + 16 * a + c16, t.M - 1), j = min(wc + 16 * b + Mfma<T>::drow(lane, r), t.N - 1);
+        C[a][b][r] = L[t.c_off + i + j * ld];
+        acc[a][b][r] = (T)0;
       }
-  // one 64 x 64 x 64 product of LDS-staged halves into acc (fa rows wr..,
-  // fb rows wc.. of Bsrc, chunks c of the half)
-  auto mma_half = [&](acc_t (&acc)[2][2], T (*Asrc)[64][KP], T (*Bsrc)[64][KP]) {
+  // loader of a chunk: VEC rows from lr on, columns lk + 16 / NV * v
+  const int lr = (tid % RG) * VEC, lk = tid / RG;
+  const T* const Xr = L + t.xr_off + min(lr, t.M - 1) + lk * ld;
+  const T* const Xk = L + t.xk_off + min(lr, t.N - 1) + lk * ld;
+  T* const sA = As + lk * LDR + lr;
+  vec_t ra[4][NV], rb[4][NV], iv[2][NI];
+  auto fetch = [&](int c, int k0) {  // chunk c of the block of columns from k0 on
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-      T fa0[TK / 4], fa1[TK / 4], fb0[TK / 4], fb1[TK / 4];
-#pragma unroll
-      for (int s2 = 0; s2 < TK / 4; s2++) {
-        fa0[s2] = Asrc[c][wr + c16][g * (TK / 4) + s2];
-        fa1[s2] = Asrc[c][wr + 16 + c16][g * (TK / 4) + s2];
-        fb0[s2] = Bsrc[c][wc + c16][g * (TK / 4) + s2];
-        fb1[s2] = Bsrc[c][wc + 16 + c16][g * (TK / 4) + s2];
-      }
-#pragma unroll
-      for (int s2 = 0; s2 < TK / 4; s2++) {
-        acc[0][0] = Mfma<T>::step(fb0[s2], fa0[s2], acc[0][0]);
-        acc[0][1] = Mfma<T>::step(fb1[s2], fa0[s2], acc[0][1]);
-        acc[1][0] = Mfma<T>::step(fb0[s2], fa1[s2], acc[1][0]);
-        acc[1][1] = Mfma<T>::step(fb1[s2], fa1[s2], acc[1][1]);
-      }
+    for (int v = 0; v < NV; v++) {
+      const long long o = (k0 + 16 * c + 16 / NV * v) * ld;
+      ra[c][v] = *(const vecu_t*)(Xr + o);
+      rb[c][v] = *(const vecu_t*)(Xk + o);
     }
   };
-  // a matrix in the accumulator layout into As, half h (its columns 32h..32h+31
-  // are held by the waves with wc == 32h), as the A operand's chunks
-  auto stage_acc = [&](const acc_t (&M)[2][2], int h) {
-    if (wc == 32 * h) {
+  // half h of the inverse: rows ij + 256 / (32 / VEC) * q, columns 32 h + ik ..
+  const int ik = (tid % (32 / VEC)) * VEC, ij = tid / (32 / VEC);
+  auto fetch_inv = [&](int h, int q) {
+    iv[h][q] = *(const vec_t*)(Inv + t.inv_off + (ij + 8 * VEC * q) * 64 + 32 * h + ik);
+  };
+  // chunk c into its buffer (A and B alternate)
+  auto stash = [&](int c, int v) {
+    asm volatile("" : "+v"(ra[c][v]));
+    asm volatile("" : "+v"(rb[c][v]));
+    T* const d = sA + ((c & 1) * 32 + 16 / NV * v) * LDR;
+    *(vec_t*)d = ra[c][v];
+    *(vec_t*)(d + 16 * LDR) = rb[c][v];
+  };
+  T fa[2][2], fb[2][2];
+  // the 4 MFMAs of step s, op(m) behind the m-th
+  auto step = [&](acc_t (&ac)[2][2], int s, auto&& op) {
 #pragma unroll
-      for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) As[b][wr + 16 * a + c16][Mfma<T>::drow(lane, r)] = M[a][b][r];
+    for (int m = 0; m < 4; m++) {
+      ac[m >> 1][m & 1] = Mfma<T>::step(fb[s & 1][m & 1], fa[s & 1][m >> 1], ac[m >> 1][m & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      op(m);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  acc_t acc[2][2];
+  // C -= Xr Xk^T over the earlier blocks
+  if (t.kpre == 0) {
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+    for (int h = 0; h < 2; h++)
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc[a][b][r] = (T)0;
-  // the inverse in the loader layout: loaded into rb once the last earlier
-  // block is staged (at once without earlier blocks)
-  T ra[4][TK / 4], rb[4][TK / 4];
-  auto fetch_inv = [&]() {
-#pragma unroll
-    for (int ch = 0; ch < 4; ch++)
-#pragma unroll
-      for (int q = 0; q < TK / 4; q++) {
-        const int k = ch * TK + lk + 4 * q;
-        rb[ch][q] = (li < t.N && k < t.N) ? Inv[t.inv_off + li * 64 + k] : (T)0;
-      }
-  };
-  // C -= Xr Xk^T over the earlier blocks, 64 columns at a time, the next
-  // block's loads issued before the current block's second half
-  if (t.kpre == 0) fetch_inv();
-  if (t.kpre > 0) {
-    auto fetch = [&](int k0) {
-#pragma unroll
-      for (int ch = 0; ch < 4; ch++)
-#pragma unroll
-        for (int q = 0; q < TK / 4; q++) {
-          const long long k = k0 + ch * TK + lk + 4 * q;
-          ra[ch][q] = li < t.M ? L[t.xr_off + li + k * ld] : (T)0;
-          rb[ch][q] = li < t.N ? L[t.xk_off + li + k * ld] : (T)0;
-        }
+      for (int q = 0; q < NI; q++) fetch_inv(h, q);
+  } else {
+    // fragment m of step s of chunk c
+    auto frag = [&](int c, int s, int m) {
+      const T* const p = As + ((c & 1) * 32 + 4 * g + s) * LDR + c16;
+      if (m < 2) fa[s & 1][m] = p[wr + 16 * m];
+      else fb[s & 1][m - 2] = p[16 * LDR + wc + 16 * (m - 2)];
     };
-    fetch(0);
+#pragma unroll
+    for (int c = 0; c < 4; c++) fetch(c, 0);
+#pragma unroll
+    for (int v = 0; v < NV; v++) stash(0, v);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 4; m++) frag(0, 0, m);
     for (int k0 = 0; k0 < t.kpre; k0 += 64) {
+      const bool more = k0 + 64 < t.kpre;
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        __syncthreads();  // the previous half's fragments are read
+      for (int c = 0; c < 4; c++) {
+        // the registers of chunk c were stored one chunk ago: they take the
+        // next block's chunk, or after the last block the inverse
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+          fetch(c, k0 + 64);
+        } else {
 #pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-          for (int q = 0; q < TK / 4; q++) {
-            As[c][li][lk + 4 * q] = ra[2 * h + c][q];
-            Bs[c][li][lk + 4 * q] = rb[2 * h + c][q];
-          }
-        if (h == 1) {
-          if (k0 + 64 < t.kpre) fetch(k0 + 64);
-          else fetch_inv();
+          for (int q = 0; q < NI / 2; q++) fetch_inv(c >> 1, (c & 1) * (NI / 2) + q);
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 3; s++)
+          step(acc, s, [&](int m) {
+            frag(c, s + 1, m);
+            if (m == 3 && s >= 3 - NV && (c < 3 || more)) stash((c + 1) & 3, s - (3 - NV));
+          });
+        // the chunk's fragments are read and the next chunk is stored
         __syncthreads();
-        mma_half(acc, As, Bs);
+        __builtin_amdgcn_sched_barrier(0);
+        step(acc, 3, [&](int m) {
+          if (c < 3 || more) frag((c + 1) & 3, 0, m);
+        });
       }
     }
   }
+  // a matrix in the accumulator layout into As, [column][row]
+  auto stage_acc = [&](const acc_t (&M)[2][2]) {
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          As[(wc + 16 * b + Mfma<T>::drow(lane, r)) * LDR + wr + 16 * a + c16] = M[a][b][r];
+  };
 #pragma unroll
   for (int a = 0; a < 2; a++)
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) C[a][b][r] -= acc[a][b][r];
-  // X = C inv^T
+      for (int r = 0; r < 4; r++) {
+        const T v = C[a][b][r] - acc[a][b][r];
+        C[a][b][r] = wc + 16 * b + Mfma<T>::drow(lane, r) < t.N ? v : (T)0;
+        acc[a][b][r] = (T)0;
+      }
+  // X = C inv^T, half the inverse at a time
+  T* const Bi = As + 64 * LDR;
+  stage_acc(C);
   acc_t X[2][2];
 #pragma unroll
   for (int a = 0; a < 2; a++)
@@ -1993,14 +2106,23 @@ __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict
       for (int r = 0; r < 4; r++) X[a][b][r] = (T)0;
 #pragma unroll
   for (int h = 0; h < 2; h++) {
-    __syncthreads();
-    stage_acc(C, h);
+    // step s of the half: k = 32 h + 16 (s / 4) + 4 g + s % 4
+    auto frag = [&](int s, int m) {
+      const int k = 16 * (s >> 2) + 4 * g + (s & 3);
+      if (m < 2) fa[s & 1][m] = As[(32 * h + k) * LDR + wr + 16 * m + c16];
+      else fb[s & 1][m - 2] = Bi[(wc + 16 * (m - 2) + c16) * LDK + k];
+    };
+    if (h) __syncthreads();  // the first half's fragments are read
 #pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-      for (int q = 0; q < TK / 4; q++) Bs[c][li][lk + 4 * q] = rb[2 * h + c][q];
+    for (int q = 0; q < NI; q++) *(vec_t*)(Bi + (ij + 8 * VEC * q) * LDK + ik) = iv[h][q];
     __syncthreads();
-    mma_half(X, As, Bs);
+#pragma unroll
+    for (int m = 0; m < 4; m++) frag(0, m);
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+      step(X, s, [&](int m) {
+        if (s < 7) frag(s + 1, m);
+      });
   }
 #pragma unroll
   for (int a = 0; a < 2; a++)
@@ -2027,25 +2149,29 @@ __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict
         const int j = min(wc + 16 * b + Mfma<T>::drow(lane, r), t.Md - 1);
         dv[a][b][r] = L[t.d_off + i + j * ld];
       }
+  __syncthreads();  // the solve's fragments are read
+  stage_acc(X);
+  __syncthreads();
+  {
+    auto frag = [&](int s, int m) {
+      const T* const p = As + (16 * (s >> 2) + 4 * g + (s & 3)) * LDR + c16;
+      if (m < 2) fa[s & 1][m] = p[wr + 16 * m];
+      else fb[s & 1][m - 2] = p[wc + 16 * (m - 2)];
+    };
+#pragma unroll
+    for (int m = 0; m < 4; m++) frag(0, m);
+#pragma unroll
+    for (int s = 0; s < 16; s++)
+      step(acc, s, [&](int m) {
+        if (s < 15) frag(s + 1, m);
+      });
+  }
 #pragma unroll
   for (int a = 0; a < 2; a++)
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) asm volatile("" : "+v"(dv[a][b][r]));
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc[a][b][r] = (T)0;
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    __syncthreads();
-    stage_acc(X, h);
-    __syncthreads();
-    mma_half(acc, As, As);
-  }
   const bool pf = t.pf_front >= 0;
   T* const PA = reinterpret_cast<T*>(smem);
   T* const pdg = PA + 64 * PM_LDA + 64;
