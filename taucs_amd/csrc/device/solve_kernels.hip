@@ -433,43 +433,48 @@ __global__ __launch_bounds__(256) void k_bwd_step(const FrontDesc* __restrict__ 
 #define YS 17
 
 // Vl[i*YS + r] <- V[col + r*ldv] for i < nv, r < nrhs (0 elsewhere in the
-// 64 x 16 block), awaiting each value; all of a thread's loads are issued
-// before it waits for any.  Thread t handles row i = t & 63 (right-hand
-// sides t/64 + 4k), whose global column `col` the caller has loaded ahead.
+// 64 x 16 block), awaiting each value.  Thread t handles row i = t & 63
+// (right-hand sides t/64 + 4k), whose global column `col` the caller has loaded
+// ahead.  A poll is one round trip to memory (about 1 us, past the L2s of the
+// other XCDs): all of a thread's values are polled together, and the error word
+// only every 32nd time, so that a wait ends one round trip after its last value
+// is there.  (One value after the other, each with a look at the error word, a
+// chain step of the mesh3d 60^3 root took 3.2 us with 8 right-hand sides;
+// together 3.0.)
 template <typename T, typename V>
 __device__ __forceinline__ void await_rows(T* Vl, const V* Vg, int ldv, int col, int nv, int nrhs,
                                            int* err)
 {
   typedef typename Sentinel<V>::U U;
+  const int i = threadIdx.x & 63, r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  U* const a = reinterpret_cast<U*>(const_cast<V*>(Vg + col + (long long)r0 * ldv));
   U bits[4];
-  U* adr[4];
+  // true once every value of this thread is there
+  auto poll = [&]() {
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int e = threadIdx.x + 256 * k, i = e & 63, r = e >> 6;
-    adr[k] = nullptr;
-    bits[k] = 0;
-    if (r < nrhs && i < nv) {
-      adr[k] = reinterpret_cast<U*>(const_cast<V*>(Vg + col + (long long)r * ldv));
-      bits[k] = __hip_atomic_load(adr[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
+    for (int k = 0; k < 4; k++)
+      if (r0 + 4 * k < nrhs)
+        bits[k] = __hip_atomic_load(a + 4LL * k * ldv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bool there = true;
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int e = threadIdx.x + 256 * k, i = e & 63, r = e >> 6;
-    if (adr[k]) {
-      int it = 0;
-      while (bits[k] == Sentinel<V>::bits) {
-        if (++it > SPIN_LIMIT) {
-          atomicOr(err, 1);
-          break;
-        }
-        if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-        __builtin_amdgcn_s_sleep(1);
-        bits[k] = __hip_atomic_load(adr[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < 4; k++)
+      if (r0 + 4 * k < nrhs) there = there && bits[k] != Sentinel<V>::bits;
+    return there;
+  };
+  if (r0 < nrhs && i < nv) {
+    int it = 0;
+    while (!poll()) {
+      if (++it > SPIN_LIMIT) {
+        atomicOr(err, 1);
+        break;
       }
+      if ((it & 31) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+      __builtin_amdgcn_s_sleep(1);
     }
-    Vl[i * YS + r] = adr[k] ? (T)__builtin_bit_cast(V, bits[k]) : (T)0;
   }
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    Vl[i * YS + r0 + 4 * k] = r0 + 4 * k < nrhs && i < nv ? (T)__builtin_bit_cast(V, bits[k]) : (T)0;
 }
 
 // Y (n x nrhs, ld n) and x (rows < n of n x nrhs, ld ldx) <- the pattern;
