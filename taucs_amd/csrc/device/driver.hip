@@ -47,8 +47,8 @@ template <typename T> __global__ void k_bwd_gather(const FrontDesc*, const Panel
 template <typename T> __global__ void k_bwd_cols(const FrontDesc*, const PanelTask*, const T*, const T*, T*, int);
 template <typename T> __global__ void k_bwd_step(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, T*, int, double*, int, int);
 template <typename T> __global__ void k_sweep_clear(T*, double*, int, int, int, int*, int);
-template <typename T> __global__ void k_fwd_chain(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, T*, T*, int, int*, int*, int);
-template <typename T> __global__ void k_bwd_chain(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, const T*, int, const T*, double*, int, int*, int*, int);
+template <typename T, int NSET> __global__ void k_fwd_chain(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, T*, T*, int, int*, int*, int);
+template <typename T, int NSET> __global__ void k_bwd_chain(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, const T*, int, const T*, double*, int, int*, int*, int);
 template <typename T> __global__ void k_bwd_upd(const FrontDesc*, const PanelTask*, const int*, const T*, const double*, int, T*, int);
 template <typename T, int NR> __global__ void k_fwd_small(const FrontDesc*, const PanelTask*, int, const int*, const T*, const T*, T*, T*, int, int);
 template <typename T, int NR> __global__ void k_bwd_small(const FrontDesc*, const PanelTask*, int, const int*, const T*, const T*, const T*, int, double*, int, int);
@@ -1649,14 +1649,23 @@ static int emit_solve(tamd_dev* D, Emitter& E, const SolveBufs& sb, int n, int n
         EMIT(0, true, k_sweep_clear<T>, dim3(std::min(grid_for((long long)n * nrhs, 256), 4096u)),
              dim3(256), Y, dX, n, ldx, nrhs, tickets, (int)D->sync_n);
         break;
-      case SV_FCHAIN:
-        EMIT(0, true, k_fwd_chain<T>, grid, dim3(256), fr, tk, rows, L, Iv, W, Y, n,
+      case SV_FCHAIN: {
+        // as few sets of four right-hand sides as hold them (the times are at RhsTile)
+        auto k = k_fwd_chain<T, 0>;
+        if constexpr (sizeof(T) == 8)
+          k = nrhs <= 4 ? k_fwd_chain<T, 1> : nrhs <= 8 ? k_fwd_chain<T, 2> : k;
+        EMIT(0, true, k, grid, dim3(256), fr, tk, rows, L, Iv, W, Y, n,
              op.tile >= 0 ? tickets + op.tile : (int*)nullptr, err, nrhs);
         break;
-      case SV_BCHAIN:
-        EMIT(0, true, k_bwd_chain<T>, grid, dim3(256), fr, tk, rows, L, Iv, (const T*)Y, n,
+      }
+      case SV_BCHAIN: {
+        auto k = k_bwd_chain<T, 0>;
+        if constexpr (sizeof(T) == 8)
+          k = nrhs <= 4 ? k_bwd_chain<T, 1> : nrhs <= 8 ? k_bwd_chain<T, 2> : k;
+        EMIT(0, true, k, grid, dim3(256), fr, tk, rows, L, Iv, (const T*)Y, n,
              (const T*)Part, dX, ldx, op.tile >= 0 ? tickets + op.tile : (int*)nullptr, err, nrhs);
         break;
+      }
       case SV_FSMALL: {
         auto k = nrhs <= 1   ? k_fwd_small<T, 1>
                  : nrhs <= 4 ? k_fwd_small<T, 4>

@@ -496,6 +496,44 @@ __global__ void k_sweep_clear(T* __restrict__ Y, double* __restrict__ x, int n, 
     tickets[e] = 0;
 }
 
+// One wave's 16 rows of a product with a 64 x 16 right-hand-side block in LDS.
+// NSET = 0: the 16 x 16 x 4 MFMA, all 16 right-hand sides.  NSET = 1 or 2 (FP64):
+// its form of four 4 x 4 blocks, each block four of the rows and a set of four
+// right-hand sides, 16 cycles instead of 64: a chain step of few right-hand
+// sides spends a quarter (half) of the time in its two products, and the bits
+// are the same (both sum their four products as one fused multiply-add after
+// another in k order).  Solve of mesh3d 40^3 with one right-hand side: 1305 us
+// with NSET = 0, 1101 with 1; of mesh3d 60^3 with 8: 3569 and 3167 with 2.  The A operand is laid out alike: lane l holds row l % 16,
+// column l / 16.  Element e of a lane's result is row(lane, e) of the wave's
+// rows, right-hand side col(lane, e).
+template <typename T, int NSET> struct RhsTile {
+  static constexpr int NE = NSET;
+  struct acc_t {
+    T v[NSET];
+    __device__ T& operator[](int e) { return v[e]; }
+    __device__ const T& operator[](int e) const { return v[e]; }
+  };
+  static __device__ int row(int lane, int) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
+  static __device__ int col(int lane, int e) { return 4 * e + (lane & 3); }
+  // b: the block's row 4 st + lane / 16
+  static __device__ void step(T a, const T* b, int lane, acc_t& c)
+  {
+#pragma unroll
+    for (int e = 0; e < NSET; e++)
+      c.v[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b[4 * e + (lane & 3)], c.v[e], 0, 0, 0);
+  }
+};
+template <typename T> struct RhsTile<T, 0> {
+  static constexpr int NE = 4;
+  typedef typename Mfma<T>::acc_t acc_t;
+  static __device__ int row(int lane, int e) { return Mfma<T>::drow(lane, e); }
+  static __device__ int col(int lane, int) { return lane & 15; }
+  static __device__ void step(T a, const T* b, int lane, acc_t& c)
+  {
+    c = Mfma<T>::step(a, b[lane & 15], c);
+  }
+};
+
 // Forward sweep of one level (fronts with m > 64).  Task (front, tile t):
 // rows [64t, 64t+64) of the front's workspace W_f (m x nrhs, the right-hand
 // side plus the children's updates).  Tile t < nb (nb = ceil(s/64)) owns
@@ -504,11 +542,11 @@ __global__ void k_sweep_clear(T* __restrict__ Y, double* __restrict__ x, int n, 
 // and (last block only) updates the sub-diagonal rows that share its tile.
 // Tiles t >= nb hold sub-diagonal rows only: they subtract all nb blocks and
 // store the result in W_f for the parent's extend-add.
-// The products run on the 16x16x4 MFMA: wave w owns rows 16w..16w+15 of the
-// tile and right-hand sides 0..15 (those beyond nrhs are zero), A = L rows
+// The products run on the MFMA (RhsTile): wave w owns rows 16w..16w+15 of the
+// tile and all right-hand sides (those beyond nrhs are zero), A = L rows
 // (loaded one dependency ahead), B = the awaited y_j block in LDS; the sum
 // over dependencies stays in the accumulators.
-template <typename T>
+template <typename T, int NSET>
 __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__ fr,
                                                    const PanelTask* __restrict__ tasks,
                                                    const int* __restrict__ rows,
@@ -516,7 +554,9 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
                                                    const T* __restrict__ Inv, T* __restrict__ W,
                                                    T* Y, int ldy, int* ticket, int* err, int nrhs)
 {
-  typedef typename Mfma<T>::acc_t acc_t;
+  typedef RhsTile<T, NSET> R;
+  typedef typename R::acc_t acc_t;
+  constexpr int NE = R::NE;
   __shared__ T It[64 * 65];
   __shared__ T Yl[2][64 * YS];
   __shared__ int sh_task;
@@ -534,18 +574,19 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
   const T* Lf = L + d.offL;
   const int* rw = rows + d.rows;  // global column of each of the front's first s rows
   const int arow = 16 * wv + c16;
-  T w0[4];
+  T w0[NE];
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int i = 16 * wv + Mfma<T>::drow(lane, k);
-    w0[k] = (c16 < nrhs && i < nr) ? w[r0 + i + (long long)c16 * m] : (T)0;
+  for (int k = 0; k < NE; k++) {
+    const int i = 16 * wv + R::row(lane, k);
+    const int c = R::col(lane, k);
+    w0[k] = (c < nrhs && i < nr) ? w[r0 + i + (long long)c * m] : (T)0;
   }
   // global columns loaded ahead: the rows this lane publishes, and the row
   // (tid & 63) of each dependency block this thread awaits
-  int pcol[4];
+  int pcol[NE];
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int i = 16 * wv + Mfma<T>::drow(lane, k);
+  for (int k = 0; k < NE; k++) {
+    const int i = 16 * wv + R::row(lane, k);
     pcol[k] = (isblk && i < kb) ? rw[r0 + i] : 0;
   }
   if (isblk) {
@@ -554,7 +595,7 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
   }
   acc_t D0, D1;  // even and odd k steps: two independent MFMA chains
 #pragma unroll
-  for (int k = 0; k < 4; k++) D0[k] = D1[k] = (T)0;
+  for (int k = 0; k < NE; k++) D0[k] = D1[k] = (T)0;
   T lv[16];
   int dcol = 0;
   auto fetch = [&](int j) {
@@ -577,60 +618,63 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
     if (j + 1 < ndep) fetch(j + 1);
 #pragma unroll
     for (int st = 0; st < 16; st += 2) {
-      D0 = Mfma<T>::step(cur[st], yb[(4 * st + kq) * YS + c16], D0);
-      D1 = Mfma<T>::step(cur[st + 1], yb[(4 * st + 4 + kq) * YS + c16], D1);
+      R::step(cur[st], yb + (4 * st + kq) * YS, lane, D0);
+      R::step(cur[st + 1], yb + (4 * st + 4 + kq) * YS, lane, D1);
     }
   }
-  T acc[4];
+  T acc[NE];
 #pragma unroll
-  for (int k = 0; k < 4; k++) acc[k] = w0[k] - (D0[k] + D1[k]);
+  for (int k = 0; k < NE; k++) acc[k] = w0[k] - (D0[k] + D1[k]);
   if (!isblk) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int i = 16 * wv + Mfma<T>::drow(lane, k);
-      if (c16 < nrhs && i < nr) w[r0 + i + (long long)c16 * m] = acc[k];
+    for (int k = 0; k < NE; k++) {
+      const int i = 16 * wv + R::row(lane, k);
+      const int c = R::col(lane, k);
+      if (c < nrhs && i < nr) w[r0 + i + (long long)c * m] = acc[k];
     }
     return;
   }
   // y = inv(L_tt) acc: A = inverse rows (zero beyond kb), B = acc (64 x 16)
   T* Ac = Yl[ndep & 1];  // not read since the last dependency's barrier
 #pragma unroll
-  for (int k = 0; k < 4; k++) Ac[(16 * wv + Mfma<T>::drow(lane, k)) * YS + c16] = acc[k];
+  for (int k = 0; k < NE; k++) Ac[(16 * wv + R::row(lane, k)) * YS + R::col(lane, k)] = acc[k];
   __syncthreads();
   acc_t Ya, Yb;
 #pragma unroll
-  for (int k = 0; k < 4; k++) Ya[k] = Yb[k] = (T)0;
+  for (int k = 0; k < NE; k++) Ya[k] = Yb[k] = (T)0;
 #pragma unroll
   for (int st = 0; st < 16; st += 2) {
-    Ya = Mfma<T>::step(It[arow + (4 * st + kq) * 65], Ac[(4 * st + kq) * YS + c16], Ya);
-    Yb = Mfma<T>::step(It[arow + (4 * st + 4 + kq) * 65], Ac[(4 * st + 4 + kq) * YS + c16], Yb);
+    R::step(It[arow + (4 * st + kq) * 65], Ac + (4 * st + kq) * YS, lane, Ya);
+    R::step(It[arow + (4 * st + 4 + kq) * 65], Ac + (4 * st + 4 + kq) * YS, lane, Yb);
   }
   acc_t Yd;
 #pragma unroll
-  for (int k = 0; k < 4; k++) Yd[k] = Ya[k] + Yb[k];
+  for (int k = 0; k < NE; k++) Yd[k] = Ya[k] + Yb[k];
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int i = 16 * wv + Mfma<T>::drow(lane, k);
-    if (i < kb && c16 < nrhs) publish(Y + pcol[k] + (long long)c16 * ldy, (T)Yd[k]);
+  for (int k = 0; k < NE; k++) {
+    const int i = 16 * wv + R::row(lane, k);
+    const int c = R::col(lane, k);
+    if (i < kb && c < nrhs) publish(Y + pcol[k] + (long long)c * ldy, (T)Yd[k]);
   }
   if (nr > kb) {  // sub-diagonal rows in the last block's tile: acc -= L[rows, blk t] y_t
     T* Yv = Yl[(ndep + 1) & 1];  // free since the barrier above
 #pragma unroll
-    for (int k = 0; k < 4; k++) Yv[(16 * wv + Mfma<T>::drow(lane, k)) * YS + c16] = Yd[k];
+    for (int k = 0; k < NE; k++) Yv[(16 * wv + R::row(lane, k)) * YS + R::col(lane, k)] = Yd[k];
     __syncthreads();
     acc_t D2;
 #pragma unroll
-    for (int k = 0; k < 4; k++) D2[k] = (T)0;
+    for (int k = 0; k < NE; k++) D2[k] = (T)0;
 #pragma unroll
     for (int st = 0; st < 16; st++) {
       const int k = 4 * st + kq;
       const T a = (arow < nr && k < kb) ? Lf[r0 + arow + (long long)(r0 + k) * m] : (T)0;
-      D2 = Mfma<T>::step(a, Yv[k * YS + c16], D2);
+      R::step(a, Yv + k * YS, lane, D2);
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int i = 16 * wv + Mfma<T>::drow(lane, k);
-      if (i >= kb && i < nr && c16 < nrhs) w[r0 + i + (long long)c16 * m] = acc[k] - D2[k];
+    for (int k = 0; k < NE; k++) {
+      const int i = 16 * wv + R::row(lane, k);
+      const int c = R::col(lane, k);
+      if (i >= kb && i < nr && c < nrhs) w[r0 + i + (long long)c * m] = acc[k] - D2[k];
     }
   }
 }
@@ -643,7 +687,7 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
 // is published in x.  MFMA products as in k_fwd_chain with wave w owning the
 // block's columns 16w..16w+15: A = L^T (read down the block's columns, one
 // dependency ahead), B = the awaited x_j block in LDS.
-template <typename T>
+template <typename T, int NSET>
 __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__ fr,
                                                    const PanelTask* __restrict__ tasks,
                                                    const int* __restrict__ rows,
@@ -653,7 +697,9 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
                                                    const T* __restrict__ Part, double* x,
                                                    int ldx, int* ticket, int* err, int nrhs)
 {
-  typedef typename Mfma<T>::acc_t acc_t;
+  typedef RhsTile<T, NSET> R;
+  typedef typename R::acc_t acc_t;
+  constexpr int NE = R::NE;
   __shared__ T It[64 * 65];
   __shared__ T Xl[2][64 * YS];
   __shared__ int sh_task;
@@ -667,15 +713,15 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
   const T* Lf = L + d.offL;
   const int* rw = rows + d.rows;
   const int acol = 16 * wv + c16;  // A-operand row = block column of this lane
-  T y0[4];
+  T y0[NE];
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int q = 16 * wv + Mfma<T>::drow(lane, k);
-    // slot stride 64 x nrhs: only the columns c16 < nrhs exist
+  for (int k = 0; k < NE; k++) {
+    const int q = 16 * wv + R::row(lane, k), c = R::col(lane, k);
+    // slot stride 64 x nrhs: only the columns c < nrhs exist
     const long long pst = 64LL * nrhs;
-    const T* ps = Part + (long long)t.kb * pst + q + c16 * 64;
+    const T* ps = Part + (long long)t.kb * pst + q + c * 64;
     T s0 = (T)0, s1 = (T)0, s2 = (T)0, s3 = (T)0;  // slots in four interleaved sums
-    if (c16 < nrhs) {
+    if (c < nrhs) {
       int u = 0;
       for (; u + 3 < t.nr; u += 4) {
         s0 += ps[(long long)u * pst];
@@ -686,22 +732,22 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
       for (; u < t.nr; u++) s0 += ps[(long long)u * pst];
     }
     const T sum = (s0 + s1) + (s2 + s3);
-    y0[k] = (c16 < nrhs && q < kb) ? Y[rw[c0 + q] + (long long)c16 * ldy] - sum : (T)0;
+    y0[k] = (c < nrhs && q < kb) ? Y[rw[c0 + q] + (long long)c * ldy] - sum : (T)0;
   }
   {
     const T* iv = Inv + d.offI + (long long)blk * 4096;
     for (int e = tid; e < 4096; e += 256) It[(e >> 6) + (e & 63) * 65] = iv[e];
   }
   const int ndep = nb - 1 - blk;  // blocks nb-1 down to blk+1
-  int pcol[4];  // the columns this lane publishes, loaded ahead
+  int pcol[NE];  // the columns this lane publishes, loaded ahead
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int q = 16 * wv + Mfma<T>::drow(lane, k);
+  for (int k = 0; k < NE; k++) {
+    const int q = 16 * wv + R::row(lane, k);
     pcol[k] = q < kb ? rw[c0 + q] : 0;
   }
   acc_t D0, D1;  // even and odd k steps: two independent MFMA chains
 #pragma unroll
-  for (int k = 0; k < 4; k++) D0[k] = D1[k] = (T)0;
+  for (int k = 0; k < NE; k++) D0[k] = D1[k] = (T)0;
   T lv[16];
   int dcol = 0;
   auto fetch = [&](int u) {
@@ -725,28 +771,29 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
     if (u + 1 < ndep) fetch(u + 1);
 #pragma unroll
     for (int st = 0; st < 16; st += 2) {
-      D0 = Mfma<T>::step(cur[st], xb[(4 * st + kq) * YS + c16], D0);
-      D1 = Mfma<T>::step(cur[st + 1], xb[(4 * st + 4 + kq) * YS + c16], D1);
+      R::step(cur[st], xb + (4 * st + kq) * YS, lane, D0);
+      R::step(cur[st + 1], xb + (4 * st + 4 + kq) * YS, lane, D1);
     }
   }
   T* Z = Xl[ndep & 1];  // not read since the last dependency's barrier
 #pragma unroll
-  for (int k = 0; k < 4; k++)
-    Z[(16 * wv + Mfma<T>::drow(lane, k)) * YS + c16] = y0[k] - (D0[k] + D1[k]);
+  for (int k = 0; k < NE; k++)
+    Z[(16 * wv + R::row(lane, k)) * YS + R::col(lane, k)] = y0[k] - (D0[k] + D1[k]);
   __syncthreads();
   // x = inv(L_bb)^T z: A[q][p] = inv(p, q)
   acc_t Xa, Xb;
 #pragma unroll
-  for (int k = 0; k < 4; k++) Xa[k] = Xb[k] = (T)0;
+  for (int k = 0; k < NE; k++) Xa[k] = Xb[k] = (T)0;
 #pragma unroll
   for (int st = 0; st < 16; st += 2) {
-    Xa = Mfma<T>::step(It[(4 * st + kq) + acol * 65], Z[(4 * st + kq) * YS + c16], Xa);
-    Xb = Mfma<T>::step(It[(4 * st + 4 + kq) + acol * 65], Z[(4 * st + 4 + kq) * YS + c16], Xb);
+    R::step(It[(4 * st + kq) + acol * 65], Z + (4 * st + kq) * YS, lane, Xa);
+    R::step(It[(4 * st + 4 + kq) + acol * 65], Z + (4 * st + 4 + kq) * YS, lane, Xb);
   }
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int q = 16 * wv + Mfma<T>::drow(lane, k);
-    if (q < kb && c16 < nrhs) publish(x + pcol[k] + (long long)c16 * ldx, (double)(Xa[k] + Xb[k]));
+  for (int k = 0; k < NE; k++) {
+    const int q = 16 * wv + R::row(lane, k);
+    const int c = R::col(lane, k);
+    if (q < kb && c < nrhs) publish(x + pcol[k] + (long long)c * ldx, (double)(Xa[k] + Xb[k]));
   }
 }
 
@@ -928,6 +975,12 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
                                               const T*, const T*, T*, T*, int, int);            \
   template __global__ void k_bwd_small<T, NR>(const FrontDesc*, const PanelTask*, int, const int*, \
                                               const T*, const T*, const T*, int, double*, int, int);
+#define CHAIN_INST(T, NSET)                                                                     \
+  template __global__ void k_fwd_chain<T, NSET>(const FrontDesc*, const PanelTask*, const int*, \
+                                                const T*, const T*, T*, T*, int, int*, int*, int); \
+  template __global__ void k_bwd_chain<T, NSET>(const FrontDesc*, const PanelTask*, const int*, \
+                                                const T*, const T*, const T*, int, const T*,    \
+                                                double*, int, int*, int*, int);
 #define TAMD_SINST(T)                                                                           \
   template __global__ void k_solve_init<T>(const FrontDesc*, const PanelTask*, int, const int*,  \
                                            const double*, int, T*, int);                        \
@@ -948,15 +1001,13 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
   template __global__ void k_bwd_step<T>(const FrontDesc*, const PanelTask*, const int*,         \
                                          const T*, const T*, T*, int, double*, int, int);       \
   template __global__ void k_sweep_clear<T>(T*, double*, int, int, int, int*, int);           \
-  template __global__ void k_fwd_chain<T>(const FrontDesc*, const PanelTask*, const int*,        \
-                                          const T*, const T*, T*, T*, int, int*, int*, int);    \
-  template __global__ void k_bwd_chain<T>(const FrontDesc*, const PanelTask*, const int*,        \
-                                          const T*, const T*, const T*, int, const T*, double*, \
-                                          int, int*, int*, int);                                \
+  CHAIN_INST(T, 0)                                                                              \
   template __global__ void k_bwd_upd<T>(const FrontDesc*, const PanelTask*, const int*, const T*, \
                                         const double*, int, T*, int);                          \
   SMALL_INST(T, 1) SMALL_INST(T, 4) SMALL_INST(T, 8) SMALL_INST(T, 16)
 TAMD_SINST(double)
+CHAIN_INST(double, 1)
+CHAIN_INST(double, 2)
 TAMD_SINST(float)
 
 }  // namespace tamd
