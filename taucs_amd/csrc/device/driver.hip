@@ -1650,18 +1650,14 @@ static int emit_solve(tamd_dev* D, Emitter& E, const SolveBufs& sb, int n, int n
              dim3(256), Y, dX, n, ldx, nrhs, tickets, (int)D->sync_n);
         break;
       case SV_FCHAIN: {
-        // as few sets of four right-hand sides as hold them (the times are at RhsTile)
-        auto k = k_fwd_chain<T, 0>;
-        if constexpr (sizeof(T) == 8)
-          k = nrhs <= 4 ? k_fwd_chain<T, 1> : nrhs <= 8 ? k_fwd_chain<T, 2> : k;
+        // as few sets of four right-hand sides as hold them (RhsTile has the times)
+        auto k = nrhs <= 4 ? k_fwd_chain<T, 1> : nrhs <= 8 ? k_fwd_chain<T, 2> : k_fwd_chain<T, 4>;
         EMIT(0, true, k, grid, dim3(256), fr, tk, rows, L, Iv, W, Y, n,
              op.tile >= 0 ? tickets + op.tile : (int*)nullptr, err, nrhs);
         break;
       }
       case SV_BCHAIN: {
-        auto k = k_bwd_chain<T, 0>;
-        if constexpr (sizeof(T) == 8)
-          k = nrhs <= 4 ? k_bwd_chain<T, 1> : nrhs <= 8 ? k_bwd_chain<T, 2> : k;
+        auto k = nrhs <= 4 ? k_bwd_chain<T, 1> : nrhs <= 8 ? k_bwd_chain<T, 2> : k_bwd_chain<T, 4>;
         EMIT(0, true, k, grid, dim3(256), fr, tk, rows, L, Iv, (const T*)Y, n,
              (const T*)Part, dX, ldx, op.tile >= 0 ? tickets + op.tile : (int*)nullptr, err, nrhs);
         break;

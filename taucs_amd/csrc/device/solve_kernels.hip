@@ -429,10 +429,96 @@ __global__ __launch_bounds__(256) void k_bwd_step(const FrontDesc* __restrict__ 
 // (Sentinel<T>, publish: the readiness protocol, in kernels.h)
 
 // Right-hand-side blocks of the chained kernels live in LDS as 64 x 16
-// arrays [row][rhs] with row stride YS (padded against bank conflicts).
+// arrays [row][rhs], their rows padded against bank conflicts (YS: k_bwd_upd's).
 #define YS 17
 
-// Vl[i*YS + r] <- V[col + r*ldv] for i < nv, r < nrhs (0 elsewhere in the
+// One wave's 16 rows of a product with a 64 x 16 right-hand-side block in LDS,
+// in NSET sets of four right-hand sides (1, 2 or 4), on the MFMAs made of 4 x 4
+// blocks: FP64 4 x 4 x 4, four blocks = 16 rows, 16 cycles a set; FP32 4 x 4 x 1,
+// sixteen blocks = 16 rows at four k, 8 cycles a set.  Four sets cost what the
+// 16 x 16 x 4 MFMA costs (64 and 32 cycles), so a chain step of few right-hand
+// sides spends a quarter (half) of that in its two products; four FP64 sets are
+// that MFMA, which reads one value of the block where they read four.  The order of
+// summation does not depend on NSET, so a column's bits do not depend on how many
+// columns there are: FP64 sums along k one after the other (as the 16 x 16 x 4
+// MFMA does), FP32 the four residues of k mod 4 apart, which sum() adds in pairs.
+// The A operand: lane l holds row l % 16, column l / 16.  Result e of a lane is
+// row(lane, e) of the wave's rows, right-hand side col(lane, e).  A row of the block
+// has LD values, right-hand side r at pos(r), so that a lane's sets are one load.
+// Measured against the 16 x 16 x 4 MFMA: FP64 solve of mesh3d 40^3 with one
+// right-hand side 1305 -> 1101 us, of mesh3d 60^3 with 8 3569 -> 3167; FP32, with
+// the copies to and from the host, of mesh3d 40^3 with 1, 8 and 16 1206 -> 1082,
+// 1806 -> 1625 and 2652 -> 2526.  (With a row's right-hand sides in order, four
+// loads a step, 12 and 16 were slower than on the 16 x 16 x 4: 2332 and 2696.)
+template <typename T, int NSET> struct RhsTile {
+  typedef typename std::conditional<sizeof(T) == 8, double, f4_t>::type set_t;
+  typedef T sets_t __attribute__((ext_vector_type(NSET)));
+  struct acc_t { set_t v[NSET]; };
+  static constexpr int LD = sizeof(T) == 8 ? 18 : 20;  // 16-byte rows, padded against bank conflicts
+  static __device__ int pos(int r) { return 4 * (r & 3) + (r >> 2); }
+  static __device__ int row(int lane, int) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
+  static __device__ int col(int lane, int e) { return 4 * e + (lane & 3); }
+  static __device__ void zero(acc_t& c)
+  {
+#pragma unroll
+    for (int e = 0; e < NSET; e++) c.v[e] = set_t{};
+  }
+  // c += A(:, 4 st .. 4 st + 3) x the block's rows 4 st ..; b: row 4 st + lane / 16
+  static __device__ void step(T a, const T* b, int lane, acc_t& c)
+  {
+    const sets_t bs = *reinterpret_cast<const sets_t*>(b + 4 * (lane & 3));
+#pragma unroll
+    for (int e = 0; e < NSET; e++)
+      if constexpr (sizeof(T) == 8)
+        c.v[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, bs[e], c.v[e], 0, 0, 0);
+      else
+        c.v[e] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, bs[e], c.v[e], 0, 0, 0);
+  }
+  // out[e] = the lane's element of c + d, set e
+  static __device__ void sum(const acc_t& c, const acc_t& d, T* out)
+  {
+#pragma unroll
+    for (int e = 0; e < NSET; e++)
+      if constexpr (sizeof(T) == 8) {
+        out[e] = c.v[e] + d.v[e];
+      } else {
+        // register i of a lane: row 4 * (lane / 4 % 4) + i, the k = lane / 16 mod 4;
+        // two exchanges add the four k and leave row i with the lanes 16 i ..
+        const f4_t v = c.v[e] + d.v[e];
+        const float lo = swap_add<32>(v[0], v[2]), hi = swap_add<32>(v[1], v[3]);
+        out[e] = swap_add<16>(lo, hi);
+      }
+  }
+  // lanes with bit N of the lane number clear: x + x of the lane N further;
+  // the others: y + y of the lane N before
+  template <int N> static __device__ float swap_add(float x, float y)
+  {
+    const auto r = N == 32
+        ? __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false)
+        : __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+};
+
+template <> struct RhsTile<double, 4> {
+  struct acc_t { d4_t v; };
+  static constexpr int LD = 17;
+  static __device__ int pos(int r) { return r; }
+  static __device__ int row(int lane, int e) { return Mfma<double>::drow(lane, e); }
+  static __device__ int col(int lane, int) { return lane & 15; }
+  static __device__ void zero(acc_t& c) { c.v = d4_t{}; }
+  static __device__ void step(double a, const double* b, int lane, acc_t& c)
+  {
+    c.v = Mfma<double>::step(a, b[lane & 15], c.v);
+  }
+  static __device__ void sum(const acc_t& c, const acc_t& d, double* out)
+  {
+#pragma unroll
+    for (int e = 0; e < 4; e++) out[e] = c.v[e] + d.v[e];
+  }
+};
+
+// Vl[i*R::LD + R::pos(r)] <- V[col + r*ldv] for i < nv, r < nrhs (0 elsewhere in the
 // 64 x 16 block), awaiting each value.  Thread t handles row i = t & 63
 // (right-hand sides t/64 + 4k), whose global column `col` the caller has loaded
 // ahead.  A poll is one round trip to memory (about 1 us, past the L2s of the
@@ -441,7 +527,7 @@ __global__ __launch_bounds__(256) void k_bwd_step(const FrontDesc* __restrict__ 
 // is there.  (One value after the other, each with a look at the error word, a
 // chain step of the mesh3d 60^3 root took 3.2 us with 8 right-hand sides;
 // together 3.0.)
-template <typename T, typename V>
+template <typename R, typename T, typename V>
 __device__ __forceinline__ void await_rows(T* Vl, const V* Vg, int ldv, int col, int nv, int nrhs,
                                            int* err)
 {
@@ -474,7 +560,8 @@ __device__ __forceinline__ void await_rows(T* Vl, const V* Vg, int ldv, int col,
   }
 #pragma unroll
   for (int k = 0; k < 4; k++)
-    Vl[i * YS + r0 + 4 * k] = r0 + 4 * k < nrhs && i < nv ? (T)__builtin_bit_cast(V, bits[k]) : (T)0;
+    Vl[i * R::LD + R::pos(r0 + 4 * k)] =
+        r0 + 4 * k < nrhs && i < nv ? (T)__builtin_bit_cast(V, bits[k]) : (T)0;
 }
 
 // Y (n x nrhs, ld n) and x (rows < n of n x nrhs, ld ldx) <- the pattern;
@@ -495,44 +582,6 @@ __global__ void k_sweep_clear(T* __restrict__ Y, double* __restrict__ x, int n, 
   for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < nt; e += gridDim.x * blockDim.x)
     tickets[e] = 0;
 }
-
-// One wave's 16 rows of a product with a 64 x 16 right-hand-side block in LDS.
-// NSET = 0: the 16 x 16 x 4 MFMA, all 16 right-hand sides.  NSET = 1 or 2 (FP64):
-// its form of four 4 x 4 blocks, each block four of the rows and a set of four
-// right-hand sides, 16 cycles instead of 64: a chain step of few right-hand
-// sides spends a quarter (half) of the time in its two products, and the bits
-// are the same (both sum their four products as one fused multiply-add after
-// another in k order).  Solve of mesh3d 40^3 with one right-hand side: 1305 us
-// with NSET = 0, 1101 with 1; of mesh3d 60^3 with 8: 3569 and 3167 with 2.  The A operand is laid out alike: lane l holds row l % 16,
-// column l / 16.  Element e of a lane's result is row(lane, e) of the wave's
-// rows, right-hand side col(lane, e).
-template <typename T, int NSET> struct RhsTile {
-  static constexpr int NE = NSET;
-  struct acc_t {
-    T v[NSET];
-    __device__ T& operator[](int e) { return v[e]; }
-    __device__ const T& operator[](int e) const { return v[e]; }
-  };
-  static __device__ int row(int lane, int) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
-  static __device__ int col(int lane, int e) { return 4 * e + (lane & 3); }
-  // b: the block's row 4 st + lane / 16
-  static __device__ void step(T a, const T* b, int lane, acc_t& c)
-  {
-#pragma unroll
-    for (int e = 0; e < NSET; e++)
-      c.v[e] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b[4 * e + (lane & 3)], c.v[e], 0, 0, 0);
-  }
-};
-template <typename T> struct RhsTile<T, 0> {
-  static constexpr int NE = 4;
-  typedef typename Mfma<T>::acc_t acc_t;
-  static __device__ int row(int lane, int e) { return Mfma<T>::drow(lane, e); }
-  static __device__ int col(int lane, int) { return lane & 15; }
-  static __device__ void step(T a, const T* b, int lane, acc_t& c)
-  {
-    c = Mfma<T>::step(a, b[lane & 15], c);
-  }
-};
 
 // Forward sweep of one level (fronts with m > 64).  Task (front, tile t):
 // rows [64t, 64t+64) of the front's workspace W_f (m x nrhs, the right-hand
@@ -556,9 +605,8 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
 {
   typedef RhsTile<T, NSET> R;
   typedef typename R::acc_t acc_t;
-  constexpr int NE = R::NE;
   __shared__ T It[64 * 65];
-  __shared__ T Yl[2][64 * YS];
+  __shared__ alignas(16) T Yl[2][64 * R::LD];
   __shared__ int sh_task;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c16 = lane & 15, kq = lane >> 4;
   if (tid == 0) sh_task = ticket ? atomicAdd(ticket, 1) : (int)blockIdx.x;
@@ -574,18 +622,18 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
   const T* Lf = L + d.offL;
   const int* rw = rows + d.rows;  // global column of each of the front's first s rows
   const int arow = 16 * wv + c16;
-  T w0[NE];
+  T w0[NSET];
 #pragma unroll
-  for (int k = 0; k < NE; k++) {
+  for (int k = 0; k < NSET; k++) {
     const int i = 16 * wv + R::row(lane, k);
     const int c = R::col(lane, k);
     w0[k] = (c < nrhs && i < nr) ? w[r0 + i + (long long)c * m] : (T)0;
   }
   // global columns loaded ahead: the rows this lane publishes, and the row
   // (tid & 63) of each dependency block this thread awaits
-  int pcol[NE];
+  int pcol[NSET];
 #pragma unroll
-  for (int k = 0; k < NE; k++) {
+  for (int k = 0; k < NSET; k++) {
     const int i = 16 * wv + R::row(lane, k);
     pcol[k] = (isblk && i < kb) ? rw[r0 + i] : 0;
   }
@@ -594,8 +642,8 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
     for (int e = tid; e < 4096; e += 256) It[(e >> 6) + (e & 63) * 65] = iv[e];
   }
   acc_t D0, D1;  // even and odd k steps: two independent MFMA chains
-#pragma unroll
-  for (int k = 0; k < NE; k++) D0[k] = D1[k] = (T)0;
+  R::zero(D0);
+  R::zero(D1);
   T lv[16];
   int dcol = 0;
   auto fetch = [&](int j) {
@@ -610,7 +658,7 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
   if (ndep > 0) fetch(0);
   for (int j = 0; j < ndep; j++) {
     T* yb = Yl[j & 1];
-    await_rows(yb, Y, ldy, dcol, min(64, s - 64 * j), nrhs, err);
+    await_rows<R>(yb, Y, ldy, dcol, min(64, s - 64 * j), nrhs, err);
     __syncthreads();
     T cur[16];
 #pragma unroll
@@ -618,16 +666,17 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
     if (j + 1 < ndep) fetch(j + 1);
 #pragma unroll
     for (int st = 0; st < 16; st += 2) {
-      R::step(cur[st], yb + (4 * st + kq) * YS, lane, D0);
-      R::step(cur[st + 1], yb + (4 * st + 4 + kq) * YS, lane, D1);
+      R::step(cur[st], yb + (4 * st + kq) * R::LD, lane, D0);
+      R::step(cur[st + 1], yb + (4 * st + 4 + kq) * R::LD, lane, D1);
     }
   }
-  T acc[NE];
+  T acc[NSET];
+  R::sum(D0, D1, acc);
 #pragma unroll
-  for (int k = 0; k < NE; k++) acc[k] = w0[k] - (D0[k] + D1[k]);
+  for (int k = 0; k < NSET; k++) acc[k] = w0[k] - acc[k];
   if (!isblk) {
 #pragma unroll
-    for (int k = 0; k < NE; k++) {
+    for (int k = 0; k < NSET; k++) {
       const int i = 16 * wv + R::row(lane, k);
       const int c = R::col(lane, k);
       if (c < nrhs && i < nr) w[r0 + i + (long long)c * m] = acc[k];
@@ -637,44 +686,47 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const FrontDesc* __restrict__
   // y = inv(L_tt) acc: A = inverse rows (zero beyond kb), B = acc (64 x 16)
   T* Ac = Yl[ndep & 1];  // not read since the last dependency's barrier
 #pragma unroll
-  for (int k = 0; k < NE; k++) Ac[(16 * wv + R::row(lane, k)) * YS + R::col(lane, k)] = acc[k];
+  for (int k = 0; k < NSET; k++)
+    Ac[(16 * wv + R::row(lane, k)) * R::LD + R::pos(R::col(lane, k))] = acc[k];
   __syncthreads();
   acc_t Ya, Yb;
-#pragma unroll
-  for (int k = 0; k < NE; k++) Ya[k] = Yb[k] = (T)0;
+  R::zero(Ya);
+  R::zero(Yb);
 #pragma unroll
   for (int st = 0; st < 16; st += 2) {
-    R::step(It[arow + (4 * st + kq) * 65], Ac + (4 * st + kq) * YS, lane, Ya);
-    R::step(It[arow + (4 * st + 4 + kq) * 65], Ac + (4 * st + 4 + kq) * YS, lane, Yb);
+    R::step(It[arow + (4 * st + kq) * 65], Ac + (4 * st + kq) * R::LD, lane, Ya);
+    R::step(It[arow + (4 * st + 4 + kq) * 65], Ac + (4 * st + 4 + kq) * R::LD, lane, Yb);
   }
-  acc_t Yd;
+  T Yd[NSET];
+  R::sum(Ya, Yb, Yd);
 #pragma unroll
-  for (int k = 0; k < NE; k++) Yd[k] = Ya[k] + Yb[k];
-#pragma unroll
-  for (int k = 0; k < NE; k++) {
+  for (int k = 0; k < NSET; k++) {
     const int i = 16 * wv + R::row(lane, k);
     const int c = R::col(lane, k);
-    if (i < kb && c < nrhs) publish(Y + pcol[k] + (long long)c * ldy, (T)Yd[k]);
+    if (i < kb && c < nrhs) publish(Y + pcol[k] + (long long)c * ldy, Yd[k]);
   }
   if (nr > kb) {  // sub-diagonal rows in the last block's tile: acc -= L[rows, blk t] y_t
     T* Yv = Yl[(ndep + 1) & 1];  // free since the barrier above
 #pragma unroll
-    for (int k = 0; k < NE; k++) Yv[(16 * wv + R::row(lane, k)) * YS + R::col(lane, k)] = Yd[k];
+    for (int k = 0; k < NSET; k++)
+      Yv[(16 * wv + R::row(lane, k)) * R::LD + R::pos(R::col(lane, k))] = Yd[k];
     __syncthreads();
-    acc_t D2;
-#pragma unroll
-    for (int k = 0; k < NE; k++) D2[k] = (T)0;
+    acc_t D2, zero;
+    R::zero(D2);
+    R::zero(zero);
 #pragma unroll
     for (int st = 0; st < 16; st++) {
       const int k = 4 * st + kq;
       const T a = (arow < nr && k < kb) ? Lf[r0 + arow + (long long)(r0 + k) * m] : (T)0;
-      R::step(a, Yv + k * YS, lane, D2);
+      R::step(a, Yv + k * R::LD, lane, D2);
     }
+    T d2[NSET];
+    R::sum(D2, zero, d2);
 #pragma unroll
-    for (int k = 0; k < NE; k++) {
+    for (int k = 0; k < NSET; k++) {
       const int i = 16 * wv + R::row(lane, k);
       const int c = R::col(lane, k);
-      if (i >= kb && i < nr && c < nrhs) w[r0 + i + (long long)c * m] = acc[k] - D2[k];
+      if (i >= kb && i < nr && c < nrhs) w[r0 + i + (long long)c * m] = acc[k] - d2[k];
     }
   }
 }
@@ -699,9 +751,8 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
 {
   typedef RhsTile<T, NSET> R;
   typedef typename R::acc_t acc_t;
-  constexpr int NE = R::NE;
   __shared__ T It[64 * 65];
-  __shared__ T Xl[2][64 * YS];
+  __shared__ alignas(16) T Xl[2][64 * R::LD];
   __shared__ int sh_task;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c16 = lane & 15, kq = lane >> 4;
   if (tid == 0) sh_task = ticket ? atomicAdd(ticket, 1) : (int)blockIdx.x;
@@ -713,9 +764,9 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
   const T* Lf = L + d.offL;
   const int* rw = rows + d.rows;
   const int acol = 16 * wv + c16;  // A-operand row = block column of this lane
-  T y0[NE];
+  T y0[NSET];
 #pragma unroll
-  for (int k = 0; k < NE; k++) {
+  for (int k = 0; k < NSET; k++) {
     const int q = 16 * wv + R::row(lane, k), c = R::col(lane, k);
     // slot stride 64 x nrhs: only the columns c < nrhs exist
     const long long pst = 64LL * nrhs;
@@ -739,15 +790,15 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
     for (int e = tid; e < 4096; e += 256) It[(e >> 6) + (e & 63) * 65] = iv[e];
   }
   const int ndep = nb - 1 - blk;  // blocks nb-1 down to blk+1
-  int pcol[NE];  // the columns this lane publishes, loaded ahead
+  int pcol[NSET];  // the columns this lane publishes, loaded ahead
 #pragma unroll
-  for (int k = 0; k < NE; k++) {
+  for (int k = 0; k < NSET; k++) {
     const int q = 16 * wv + R::row(lane, k);
     pcol[k] = q < kb ? rw[c0 + q] : 0;
   }
   acc_t D0, D1;  // even and odd k steps: two independent MFMA chains
-#pragma unroll
-  for (int k = 0; k < NE; k++) D0[k] = D1[k] = (T)0;
+  R::zero(D0);
+  R::zero(D1);
   T lv[16];
   int dcol = 0;
   auto fetch = [&](int u) {
@@ -763,7 +814,7 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
   for (int u = 0; u < ndep; u++) {
     const int rr0 = 64 * (nb - 1 - u);
     T* xb = Xl[u & 1];
-    await_rows(xb, x, ldx, dcol, min(64, s - rr0), nrhs, err);
+    await_rows<R>(xb, x, ldx, dcol, min(64, s - rr0), nrhs, err);
     __syncthreads();
     T cur[16];
 #pragma unroll
@@ -771,29 +822,33 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
     if (u + 1 < ndep) fetch(u + 1);
 #pragma unroll
     for (int st = 0; st < 16; st += 2) {
-      R::step(cur[st], xb + (4 * st + kq) * YS, lane, D0);
-      R::step(cur[st + 1], xb + (4 * st + 4 + kq) * YS, lane, D1);
+      R::step(cur[st], xb + (4 * st + kq) * R::LD, lane, D0);
+      R::step(cur[st + 1], xb + (4 * st + 4 + kq) * R::LD, lane, D1);
     }
   }
   T* Z = Xl[ndep & 1];  // not read since the last dependency's barrier
+  T dk[NSET];
+  R::sum(D0, D1, dk);
 #pragma unroll
-  for (int k = 0; k < NE; k++)
-    Z[(16 * wv + R::row(lane, k)) * YS + R::col(lane, k)] = y0[k] - (D0[k] + D1[k]);
+  for (int k = 0; k < NSET; k++)
+    Z[(16 * wv + R::row(lane, k)) * R::LD + R::pos(R::col(lane, k))] = y0[k] - dk[k];
   __syncthreads();
   // x = inv(L_bb)^T z: A[q][p] = inv(p, q)
   acc_t Xa, Xb;
-#pragma unroll
-  for (int k = 0; k < NE; k++) Xa[k] = Xb[k] = (T)0;
+  R::zero(Xa);
+  R::zero(Xb);
 #pragma unroll
   for (int st = 0; st < 16; st += 2) {
-    R::step(It[(4 * st + kq) + acol * 65], Z + (4 * st + kq) * YS, lane, Xa);
-    R::step(It[(4 * st + 4 + kq) + acol * 65], Z + (4 * st + 4 + kq) * YS, lane, Xb);
+    R::step(It[(4 * st + kq) + acol * 65], Z + (4 * st + kq) * R::LD, lane, Xa);
+    R::step(It[(4 * st + 4 + kq) + acol * 65], Z + (4 * st + 4 + kq) * R::LD, lane, Xb);
   }
+  T xk[NSET];
+  R::sum(Xa, Xb, xk);
 #pragma unroll
-  for (int k = 0; k < NE; k++) {
+  for (int k = 0; k < NSET; k++) {
     const int q = 16 * wv + R::row(lane, k);
     const int c = R::col(lane, k);
-    if (q < kb && c < nrhs) publish(x + pcol[k] + (long long)c * ldx, (double)(Xa[k] + Xb[k]));
+    if (q < kb && c < nrhs) publish(x + pcol[k] + (long long)c * ldx, (double)xk[k]);
   }
 }
 
@@ -1001,13 +1056,11 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
   template __global__ void k_bwd_step<T>(const FrontDesc*, const PanelTask*, const int*,         \
                                          const T*, const T*, T*, int, double*, int, int);       \
   template __global__ void k_sweep_clear<T>(T*, double*, int, int, int, int*, int);           \
-  CHAIN_INST(T, 0)                                                                              \
+  CHAIN_INST(T, 1) CHAIN_INST(T, 2) CHAIN_INST(T, 4)                                            \
   template __global__ void k_bwd_upd<T>(const FrontDesc*, const PanelTask*, const int*, const T*, \
                                         const double*, int, T*, int);                          \
   SMALL_INST(T, 1) SMALL_INST(T, 4) SMALL_INST(T, 8) SMALL_INST(T, 16)
 TAMD_SINST(double)
-CHAIN_INST(double, 1)
-CHAIN_INST(double, 2)
 TAMD_SINST(float)
 
 }  // namespace tamd

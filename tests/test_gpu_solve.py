@@ -300,14 +300,15 @@ def test_diagonal_blocks_of_every_width_class(prec, rtol):
         F.free()
 
 
+@pytest.mark.parametrize("precision", [T.FP64, T.FP32])
 @pytest.mark.parametrize("nrhs", [1, 4, 5, 8, 9])
-def test_chained_columns_do_not_depend_on_their_number(nrhs):
+def test_chained_columns_do_not_depend_on_their_number(precision, nrhs):
     """Up to four, up to eight and more right-hand sides take MFMAs of other
     shapes in the chained sweeps, which sum in the same order: a column has the
     bits that it has among sixteen."""
-    print(f"case: chained columns bitwise, mesh3d 18x17x13, nrhs {nrhs}", flush=True)
+    print(f"case: chained columns bitwise, mesh3d 18x17x13, precision {precision}, nrhs {nrhs}", flush=True)
     A = T.mesh3d(18, 17, 13)
-    F, PA = factored(A, T.FP64, True)
+    F, PA = factored(A, precision, True)
     B = np.random.default_rng(5).uniform(-1, 1, (PA.n, 16))
     X = F.solve(B)
     assert np.array_equal(F.solve(np.asfortranarray(B[:, 16 - nrhs:])), X[:, 16 - nrhs:])
