@@ -1149,7 +1149,8 @@ extern "C" long long taucs_amd_factor_device_bytes(void* vL, int precision, int 
   if (refine) {
     const long long full = 2LL * F->plan.a_nnz;
     b += 4 * (n + 1) + 12 * std::max(full, 1LL);
-    b += 6LL * 8 * n * std::max(nrhs, 1) + 8LL * (256 + 8) * std::max(nrhs, 1);
+    // the vectors, and the reductions' partials of at most 2048 blocks with the scalars
+    b += 8LL * (6 * n + 5 * std::min(2048LL, n / 256 + 1) + 4) * std::max(nrhs, 1);
   }
   return b;
 }

@@ -30,96 +30,181 @@
 
 namespace tamd {
 
-// y(:,r) = b(:,r) - A x(:,r)     (b may be null: y = A x)
-// One thread per row; A's row is read once per group of four right-hand
-// sides, and each sum runs over the row in stored order.
-__global__ void k_csr_residual(int n, const int* __restrict__ rp, const int* __restrict__ ci,
-                               const double* __restrict__ v, const double* __restrict__ x,
-                               int ldx, const double* __restrict__ b, int ldb,
-                               double* __restrict__ y, int ldy, int nrhs)
+// max that propagates NaN (fmax would drop it and hide a diverged iterate)
+__device__ __forceinline__ double maxnan(double x, double y) { return (x != x || x > y) ? x : y; }
+
+// What a residual check reduces for each column: max|r|, max|x|, max|b|, sum r^2, sum b^2
+#define NQ 5
+__device__ __forceinline__ constexpr bool is_max(int q) { return q < 3; }
+
+// The sum (or maximum) of v over the block's 256 threads, in thread 0; red: 4 values
+template <bool MAX> __device__ __forceinline__ double block_reduce(double v, double* red)
 {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int k0 = rp[i], k1 = rp[i + 1];
-  for (int r0 = 0; r0 < nrhs; r0 += 4) {
-    const int nr = nrhs - r0 < 4 ? nrhs - r0 : 4;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_down(v, off);
+    v = MAX ? maxnan(v, o) : v + o;
+  }
+  __syncthreads();  // red may still be read
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return MAX ? maxnan(maxnan(red[0], red[1]), maxnan(red[2], red[3]))
+             : (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// DOT = false: y = b - A x and the block's share of each column's NQ norms;
+// DOT = true: y = A x and the block's share of each column's x . y.
+// partial[(q * nrhs + r) * gridDim.x + block].
+// One thread per row, block column y four right-hand sides; each sum runs over
+// the row in stored order.  The norms come with the residual because r, x and b
+// are in registers here: as five reductions over memory, each of two launches and
+// a copy to the host, they cost 0.2 to 0.3 ms a check, and take 17 us now where the
+// product with A takes 90 (373 thousand rows, four right-hand sides).
+template <bool DOT>
+__global__ __launch_bounds__(256) void k_csr_residual(int n, const int* __restrict__ rp,
+                                                      const int* __restrict__ ci,
+                                                      const double* __restrict__ v,
+                                                      const double* __restrict__ x,
+                                                      const double* __restrict__ b,
+                                                      double* __restrict__ y, int nrhs,
+                                                      double* __restrict__ partial)
+{
+  __shared__ double red[4];
+  constexpr int Q = DOT ? 1 : NQ;
+  const int r0 = 4 * blockIdx.y, nr = nrhs - r0 < 4 ? nrhs - r0 : 4;
+  const double* xr = x + (long long)r0 * n;
+  double s[Q][4];
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) s[q][e] = 0.0;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int k0 = rp[i], k1 = rp[i + 1];
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    const double* xr = x + (long long)r0 * ldx;
     for (int k = k0; k < k1; k++) {
       const double a = v[k];
       const long long c = ci[k];
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (q < nr) acc[q] += a * xr[c + (long long)q * ldx];
+      for (int e = 0; e < 4; e++)
+        if (e < nr) acc[e] += a * xr[c + (long long)e * n];
     }
 #pragma unroll
-    for (int q = 0; q < 4; q++)
-      if (q < nr) {
-        const long long r = r0 + q;
-        y[i + r * ldy] = b ? b[i + r * ldb] - acc[q] : acc[q];
+    for (int e = 0; e < 4; e++)
+      if (e < nr) {
+        const long long at = i + (long long)(r0 + e) * n;
+        const double xe = x[at];
+        if constexpr (DOT) {
+          y[at] = acc[e];
+          s[0][e] += xe * acc[e];
+        } else {
+          const double be = b[at], re = be - acc[e];
+          y[at] = re;
+          s[0][e] = maxnan(s[0][e], fabs(re));
+          s[1][e] = maxnan(s[1][e], fabs(xe));
+          s[2][e] = maxnan(s[2][e], fabs(be));
+          s[3][e] += re * re;
+          s[4][e] += be * be;
+        }
       }
   }
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (e < nr) {
+        const double t = !DOT && is_max(q) ? block_reduce<true>(s[q][e], red)
+                                           : block_reduce<false>(s[q][e], red);
+        if (threadIdx.x == 0) partial[(long long)(q * nrhs + r0 + e) * gridDim.x + blockIdx.x] = t;
+      }
 }
 
-// |A| row sums (for |A|_inf)
-__global__ void k_csr_absrow(int n, const int* rp, const double* v, double* out)
+// The block's share of max_i sum_j |a_ij|  (|A|_inf)
+__global__ __launch_bounds__(256) void k_csr_absrow(int n, const int* rp, const double* v, double* partial)
 {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double acc = 0.0;
-  for (int k = rp[i]; k < rp[i + 1]; k++) acc += fabs(v[k]);
-  out[i] = acc;
-}
-
-// max that propagates NaN (fmax would drop it and hide a diverged iterate)
-__device__ __forceinline__ double maxnan(double x, double y) { return (x != x || x > y) ? x : y; }
-
-// Per-column partial reductions: mode 0 sum(a*b), 1 max|a|, 2 sum(a*a).
-// partial[(blk) + r*gridDim.x]
-__global__ __launch_bounds__(256) void k_colreduce(int n, const double* __restrict__ a, int lda,
-                                                   const double* __restrict__ b, int ldb,
-                                                   int mode, double* __restrict__ partial)
-{
-  __shared__ double red[256];
-  const int r = blockIdx.y;
-  double acc = 0.0;
+  __shared__ double red[4];
+  double m = 0.0;
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    double av = a[i + (long long)r * lda];
-    if (mode == 0) acc += av * b[i + (long long)r * ldb];
-    else if (mode == 1) acc = maxnan(acc, fabs(av));
-    else acc += av * av;
-  }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off)
-      red[threadIdx.x] = mode == 1 ? maxnan(red[threadIdx.x], red[threadIdx.x + off])
-                                   : red[threadIdx.x] + red[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x + (long long)r * gridDim.x] = red[0];
-}
-
-__global__ void k_colfinal(int nblk, int mode, const double* partial, double* out, int nrhs)
-{
-  for (int r = threadIdx.x; r < nrhs; r += blockDim.x) {
     double acc = 0.0;
-    for (int q = 0; q < nblk; q++) {
-      double v = partial[q + (long long)r * nblk];
-      acc = mode == 1 ? maxnan(acc, v) : acc + v;
-    }
-    out[r] = acc;
+    for (int k = rp[i]; k < rp[i + 1]; k++) acc += fabs(v[k]);
+    m = maxnan(m, acc);
+  }
+  m = block_reduce<true>(m, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+
+// The block's share of each column's a . b
+__global__ __launch_bounds__(256) void k_coldot(int n, const double* __restrict__ a,
+                                                const double* __restrict__ b, int nrhs,
+                                                double* __restrict__ partial)
+{
+  __shared__ double red[4];
+  const long long at = (long long)blockIdx.y * n;
+  double acc = 0.0;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) acc += a[at + i] * b[at + i];
+  acc = block_reduce<false>(acc, red);
+  if (threadIdx.x == 0) partial[(long long)blockIdx.y * gridDim.x + blockIdx.x] = acc;
+}
+
+// out[o] = the reduction of partial[o * nblk ..], o = blockIdx.x = q * nrhs + r; the
+// first nmax outputs are maxima.  One block an output: one thread an output took
+// 15 to 27 us, a chain of as many dependent additions as there are blocks.
+__global__ __launch_bounds__(256) void k_norms_final(int nblk, const double* __restrict__ partial,
+                                                     int nmax, double* __restrict__ out)
+{
+  __shared__ double red[4];
+  const int o = blockIdx.x;
+  const bool mx = o < nmax;
+  double acc = 0.0;
+  for (int q = threadIdx.x; q < nblk; q += 256) {
+    const double v = partial[(long long)o * nblk + q];
+    acc = mx ? maxnan(acc, v) : acc + v;
+  }
+  acc = mx ? block_reduce<true>(acc, red) : block_reduce<false>(acc, red);
+  if (threadIdx.x == 0) out[o] = acc;
+}
+
+// Column r's dot product d, of which
+//   CG_START:  rz = d
+//   CG_ALPHA:  scal = rz / d, 0 where d is 0 or the column is done
+//   CG_BETA:   scal = d / rz, 0 where rz is 0; rz = d
+enum { CG_START, CG_ALPHA, CG_BETA };
+__global__ __launch_bounds__(256) void k_dot_final(int nblk, const double* __restrict__ partial, int kind,
+                                                   double* rz, const int* done, double* scal)
+{
+  __shared__ double red[4];
+  const int r = blockIdx.x;
+  double d = 0.0;
+  for (int q = threadIdx.x; q < nblk; q += 256) d += partial[(long long)r * nblk + q];
+  d = block_reduce<false>(d, red);
+  if (threadIdx.x != 0) return;
+  if (kind == CG_ALPHA) {
+    scal[r] = (d != 0.0 && !done[r]) ? rz[r] / d : 0.0;
+  } else {
+    if (kind == CG_BETA) scal[r] = rz[r] != 0.0 ? d / rz[r] : 0.0;
+    rz[r] = d;
   }
 }
 
-// y(:,r) += alpha[r] * x(:,r)   (sign: +1 or -1 applied to alpha)
-__global__ void k_axpy_col(int n, const double* __restrict__ alpha, double sign,
-                           const double* __restrict__ x, double* __restrict__ y, int nrhs)
+// y(:,r) += alpha[r] * x(:,r)
+__global__ void k_axpy_col(int n, const double* __restrict__ alpha, const double* __restrict__ x,
+                           double* __restrict__ y, int nrhs)
 {
   long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (long long)n * nrhs) return;
   int r = (int)(e / n);
-  y[e] += sign * alpha[r] * x[e];
+  y[e] += alpha[r] * x[e];
+}
+
+// x += alpha p, r -= alpha q
+__global__ void k_cg_step(int n, const double* __restrict__ alpha, const double* __restrict__ p,
+                          const double* __restrict__ q, double* __restrict__ x, double* __restrict__ r,
+                          int nrhs)
+{
+  long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= (long long)n * nrhs) return;
+  const double a = alpha[(int)(e / n)];
+  x[e] += a * p[e];
+  r[e] -= a * q[e];
 }
 
 // p = z + beta p
@@ -130,13 +215,6 @@ __global__ void k_xpby_col(int n, const double* __restrict__ z, const double* __
   if (e >= (long long)n * nrhs) return;
   int r = (int)(e / n);
   p[e] = z[e] + beta[r] * p[e];
-}
-
-// out[r] = (den[r] != 0) ? num[r]/den[r] : 0, optionally masked by done[r]
-__global__ void k_ratio(const double* num, const double* den, const int* done, double* out, int nrhs)
-{
-  for (int r = threadIdx.x; r < nrhs; r += blockDim.x)
-    out[r] = (den[r] != 0.0 && !(done && done[r])) ? num[r] / den[r] : 0.0;
 }
 
 }  // namespace tamd
@@ -160,10 +238,15 @@ struct RefineCtx {
   double anorm_inf = 0.0;
   int cap = 0;  // rhs capacity of the work vectors
   double *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *x = nullptr, *b = nullptr;
-  double *partial = nullptr, *s1 = nullptr, *s2 = nullptr, *s3 = nullptr;
-  double *mask = nullptr, *rz = nullptr, *rz_new = nullptr, *scal = nullptr;
+  double *partial = nullptr, *mask = nullptr, *rz = nullptr, *scal = nullptr;
   int* done = nullptr;
+  double* norms = nullptr;  // pinned host memory: NQ x nrhs norms, then |A|_inf
 };
+
+// Blocks of the reducing kernels: one row a thread up to half a million rows
+// (eight blocks of each CU), then several.
+static constexpr int MAX_BLOCKS = 2048;
+static int row_blocks(int n) { return std::max(1, std::min(MAX_BLOCKS, (n + 255) / 256)); }
 
 struct CtxEntry { void* key; RefineCtx* ctx; };
 // Contexts of all factors; the list is shared by threads, a context is used
@@ -178,8 +261,9 @@ static void ctx_free(RefineCtx* c)
 {
   if (!c) return;
   void* ps[] = {c->rp, c->ci, c->src, c->v, c->avals, c->r, c->z, c->p, c->q, c->x, c->b, c->partial,
-                c->s1, c->s2, c->s3, c->mask, c->rz, c->rz_new, c->scal, c->done};
+                c->mask, c->rz, c->scal, c->done};
   for (void* p : ps) tamd_dev_free_ptr(p);
+  if (c->norms) (void)hipHostFree(c->norms);
   delete c;
 }
 
@@ -303,57 +387,54 @@ static RefineCtx* get_ctx(tamd_factor* F, const taucs_ccs_matrix* A, int nrhs, b
       *pp = nullptr;
       if (dmalloc(pp, sizeof(double) * (size_t)c->n * nrhs)) return nullptr;
     }
-    void** ss[] = {(void**)&c->partial, (void**)&c->s1,     (void**)&c->s2,   (void**)&c->s3,
-                   (void**)&c->mask,    (void**)&c->rz,     (void**)&c->rz_new, (void**)&c->scal,
-                   (void**)&c->done};
-    for (int i = 0; i < 9; i++) {
-      size_t sz = i == 0 ? sizeof(double) * 256 * (size_t)nrhs
-                         : (i == 8 ? sizeof(int) : sizeof(double)) * (size_t)nrhs;
-      tamd_dev_free_ptr(*ss[i]);
-      *ss[i] = nullptr;
-      if (dmalloc(ss[i], sz)) return nullptr;
+    const struct { void** p; size_t bytes; } ss[] = {
+        {(void**)&c->partial, sizeof(double) * NQ * row_blocks(c->n) * (size_t)nrhs},
+        {(void**)&c->mask, sizeof(double) * (size_t)nrhs},
+        {(void**)&c->rz, sizeof(double) * (size_t)nrhs},
+        {(void**)&c->scal, sizeof(double) * (size_t)nrhs},
+        {(void**)&c->done, sizeof(int) * (size_t)nrhs}};
+    for (const auto& e : ss) {
+      tamd_dev_free_ptr(*e.p);
+      *e.p = nullptr;
+      if (dmalloc(e.p, e.bytes)) return nullptr;
+    }
+    if (c->norms) (void)hipHostFree(c->norms);
+    c->norms = nullptr;
+    if (hipHostMalloc((void**)&c->norms, sizeof(double) * (NQ * (size_t)nrhs + 1), 0) != hipSuccess) {
+      c->norms = nullptr;
+      return nullptr;
     }
     c->cap = nrhs;
   }
   return c;
 }
 
-// out[r] = reduce over column r; blocking (returns after the stream syncs if host != null)
-static void colreduce(hipStream_t st, RefineCtx* c, const double* a, const double* b, int mode,
-                      double* dout, int nrhs)
-{
-  int nblk = std::min(256, (c->n + 255) / 256);
-  if (nblk < 1) nblk = 1;
-  hipLaunchKernelGGL(k_colreduce, dim3(nblk, nrhs), dim3(256), 0, st, c->n, a, c->n, b, c->n, mode,
-                     c->partial);
-  hipLaunchKernelGGL(k_colfinal, dim3(1), dim3(64), 0, st, nblk, mode, c->partial, dout, nrhs);
-}
-
 extern "C" int tamd_dev_stream_of(tamd_factor* F, hipStream_t* st);
 extern "C" int tamd_dev_solve_device(tamd_factor* F, int nrhs, double* dX, int ldx, const double* dB, int ldb);
 extern "C" int tamd_dev_sweep_error(tamd_factor* F);
 
-// Backward errors of x: r = b - A x,  eta = |r|_inf / (|A|_inf |x|_inf + |b|_inf)
+// Backward errors of x: r = b - A x,  eta = |r|_inf / (|A|_inf |x|_inf + |b|_inf).
+// The last kernel writes the norms to pinned host memory: one wait, no copy.
 static int residual_and_error(hipStream_t st, RefineCtx* c, const double* x, const double* b,
                               double* r, int nrhs, std::vector<double>& eta,
                               std::vector<double>& relres)
 {
-  int n = c->n;
-  hipLaunchKernelGGL(k_csr_residual, dim3((n + 255) / 256), dim3(256), 0, st, n, c->rp, c->ci, c->v, x,
-                     n, b, n, r, n, nrhs);
-  std::vector<double> rinf(nrhs), xinf(nrhs), binf(nrhs), r2(nrhs), b2(nrhs);
-  colreduce(st, c, r, nullptr, 1, c->s1, nrhs);
-  HIPOK(hipMemcpyAsync(rinf.data(), c->s1, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
-  colreduce(st, c, x, nullptr, 1, c->s2, nrhs);
-  HIPOK(hipMemcpyAsync(xinf.data(), c->s2, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
-  colreduce(st, c, b, nullptr, 1, c->s3, nrhs);
-  HIPOK(hipMemcpyAsync(binf.data(), c->s3, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
+  const int n = c->n, nblk = row_blocks(n);
+  double* const anorm = c->norms + NQ * (size_t)c->cap;
+  if (c->anorm_stale) {  // |A|_inf = max row sum of |a_ij|
+    hipLaunchKernelGGL(k_csr_absrow, dim3(nblk), dim3(256), 0, st, n, c->rp, c->v, c->partial);
+    hipLaunchKernelGGL(k_norms_final, dim3(1), dim3(256), 0, st, nblk, c->partial, 1, anorm);
+  }
+  hipLaunchKernelGGL(k_csr_residual<false>, dim3(nblk, (nrhs + 3) / 4), dim3(256), 0, st, n, c->rp, c->ci,
+                     c->v, x, b, r, nrhs, c->partial);
+  hipLaunchKernelGGL(k_norms_final, dim3(NQ * nrhs), dim3(256), 0, st, nblk, c->partial, 3 * nrhs,
+                     c->norms);
+  HIPOK(hipGetLastError());
   HIPOK(hipStreamSynchronize(st));
-  colreduce(st, c, r, nullptr, 2, c->s1, nrhs);
-  HIPOK(hipMemcpyAsync(r2.data(), c->s1, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
-  colreduce(st, c, b, nullptr, 2, c->s2, nrhs);
-  HIPOK(hipMemcpyAsync(b2.data(), c->s2, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
-  HIPOK(hipStreamSynchronize(st));
+  if (c->anorm_stale) c->anorm_inf = *anorm;
+  c->anorm_stale = false;
+  const double *rinf = c->norms, *xinf = rinf + nrhs, *binf = xinf + nrhs, *r2 = binf + nrhs,
+               *b2 = r2 + nrhs;
   eta.resize(nrhs);
   relres.resize(nrhs);
   for (int q = 0; q < nrhs; q++) {
@@ -373,13 +454,6 @@ static int refine_core(tamd_factor* F, RefineCtx* c, hipStream_t st, int nrhs, i
   const bool stop_relres = (method & TAUCS_AMD_REFINE_STOP_RELRES) != 0;
   method &= 0xff;
   int n = c->n;
-  if (c->anorm_stale) {  // |A|_inf = max row sum of |a_ij|, on the device
-    hipLaunchKernelGGL(k_csr_absrow, dim3((n + 255) / 256), dim3(256), 0, st, n, c->rp, c->v, c->r);
-    colreduce(st, c, c->r, nullptr, 1, c->s1, 1);
-    HIPOK(hipMemcpyAsync(&c->anorm_inf, c->s1, sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPOK(hipStreamSynchronize(st));
-    c->anorm_stale = false;
-  }
   if (maxit <= 0) maxit = 100;
   std::vector<double> eta, relres;
   int it = 0;
@@ -388,8 +462,8 @@ static int refine_core(tamd_factor* F, RefineCtx* c, hipStream_t st, int nrhs, i
   // Every right-hand side follows its own recurrence and stops changing once
   // its backward error reaches tol (its step is masked to zero), so a column's
   // result does not depend on which other columns are solved with it.
-  std::vector<int> done(nrhs, 0), bad(nrhs, 0), stop(nrhs, 0);
-  std::vector<double> mask(nrhs, 1.0), best(nrhs, 1e300);
+  std::vector<int> done(nrhs, 0), bad(nrhs, 0), stop(nrhs, 0), stopped(nrhs, 0);
+  std::vector<double> mask(nrhs, 1.0), best(nrhs, 1e300), sent;  // sent: the mask on the device
   // A column diverges when its residual is not finite or has grown 1000x
   // above the smallest seen: a diverging iterate can grow until |A||x|
   // dwarfs the residual, and its backward error then looks small.
@@ -415,8 +489,11 @@ static int refine_core(tamd_factor* F, RefineCtx* c, hipStream_t st, int nrhs, i
       if (settled) break;
       if (it >= maxit) break;
       if (tamd_dev_solve_device(F, nrhs, c->z, n, c->r, n)) return -1;
-      HIPOK(hipMemcpyAsync(c->mask, mask.data(), sizeof(double) * nrhs, hipMemcpyHostToDevice, st));
-      hipLaunchKernelGGL(k_axpy_col, dim3(gv), dim3(256), 0, st, n, c->mask, 1.0, c->z, c->x, nrhs);
+      if (mask != sent) {
+        HIPOK(hipMemcpyAsync(c->mask, mask.data(), sizeof(double) * nrhs, hipMemcpyHostToDevice, st));
+        sent = mask;
+      }
+      hipLaunchKernelGGL(k_axpy_col, dim3(gv), dim3(256), 0, st, n, c->mask, c->z, c->x, nrhs);
       it++;
     }
   } else {
@@ -426,15 +503,19 @@ static int refine_core(tamd_factor* F, RefineCtx* c, hipStream_t st, int nrhs, i
     if (tamd_dev_solve_device(F, nrhs, c->z, n, c->r, n)) return -1;
     HIPOK(hipMemcpyAsync(c->p, c->z, sizeof(double) * n * nrhs, hipMemcpyDeviceToDevice, st));
     HIPOK(hipMemsetAsync(c->done, 0, sizeof(int) * nrhs, st));
-    colreduce(st, c, c->r, c->z, 0, c->rz, nrhs);
+    const int nblk = row_blocks(n);
+    auto dot_final = [&](int kind) {
+      hipLaunchKernelGGL(k_dot_final, dim3(nrhs), dim3(256), 0, st, nblk, c->partial, kind, c->rz, c->done,
+                         c->scal);
+    };
+    hipLaunchKernelGGL(k_coldot, dim3(nblk, nrhs), dim3(256), 0, st, n, c->r, c->z, nrhs, c->partial);
+    dot_final(CG_START);
     for (;;) {
       // q = A p ; alpha = rz / (p.q)
-      hipLaunchKernelGGL(k_csr_residual, dim3((n + 255) / 256), dim3(256), 0, st, n, c->rp, c->ci, c->v,
-                         c->p, n, (const double*)nullptr, n, c->q, n, nrhs);
-      colreduce(st, c, c->p, c->q, 0, c->s1, nrhs);
-      hipLaunchKernelGGL(k_ratio, dim3(1), dim3(64), 0, st, c->rz, c->s1, c->done, c->scal, nrhs);
-      hipLaunchKernelGGL(k_axpy_col, dim3(gv), dim3(256), 0, st, n, c->scal, 1.0, c->p, c->x, nrhs);
-      hipLaunchKernelGGL(k_axpy_col, dim3(gv), dim3(256), 0, st, n, c->scal, -1.0, c->q, c->r, nrhs);
+      hipLaunchKernelGGL(k_csr_residual<true>, dim3(nblk, (nrhs + 3) / 4), dim3(256), 0, st, n, c->rp, c->ci,
+                         c->v, c->p, (const double*)nullptr, c->q, nrhs, c->partial);
+      dot_final(CG_ALPHA);
+      hipLaunchKernelGGL(k_cg_step, dim3(gv), dim3(256), 0, st, n, c->scal, c->p, c->q, c->x, c->r, nrhs);
       it++;
       // convergence on the true residual every iteration (k small)
       if (residual_and_error(st, c, c->x, c->b, c->q, nrhs, eta, relres)) return -1;
@@ -448,15 +529,15 @@ static int refine_core(tamd_factor* F, RefineCtx* c, hipStream_t st, int nrhs, i
       }
       if (all) { conv = true; break; }
       if (settled || it >= maxit) break;
-      HIPOK(hipMemcpyAsync(c->done, stop.data(), sizeof(int) * nrhs, hipMemcpyHostToDevice, st));
+      if (stop != stopped) {
+        HIPOK(hipMemcpyAsync(c->done, stop.data(), sizeof(int) * nrhs, hipMemcpyHostToDevice, st));
+        stopped = stop;
+      }
       if (tamd_dev_solve_device(F, nrhs, c->z, n, c->r, n)) return -1;
-      colreduce(st, c, c->r, c->z, 0, c->rz_new, nrhs);
-      hipLaunchKernelGGL(k_ratio, dim3(1), dim3(64), 0, st, c->rz_new, c->rz, (const int*)nullptr, c->scal,
-                         nrhs);
+      hipLaunchKernelGGL(k_coldot, dim3(nblk, nrhs), dim3(256), 0, st, n, c->r, c->z, nrhs, c->partial);
+      dot_final(CG_BETA);
       hipLaunchKernelGGL(k_xpby_col, dim3(gv), dim3(256), 0, st, n, c->z, c->scal, c->p, nrhs);
-      HIPOK(hipMemcpyAsync(c->rz, c->rz_new, sizeof(double) * nrhs, hipMemcpyDeviceToDevice, st));
     }
-    if (residual_and_error(st, c, c->x, c->b, c->r, nrhs, eta, relres)) return -1;
   }
   if (tamd_dev_sweep_error(F)) return -1;
   if (info) {

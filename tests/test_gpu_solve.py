@@ -313,3 +313,37 @@ def test_chained_columns_do_not_depend_on_their_number(precision, nrhs):
     X = F.solve(B)
     assert np.array_equal(F.solve(np.asfortranarray(B[:, 16 - nrhs:])), X[:, 16 - nrhs:])
     F.free()
+
+
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("mesh,nrhs", [((3, 1), 1), ((15, 17), 4), ((16, 16), 5), ((40, 29), 9),
+                                       ((727, 725), 3)])
+def test_refinement_norms_at_block_edges(method, mesh, nrhs):
+    """The residual kernel's norms: n of a few rows, one below, at and above a
+    block of 256 rows, and more rows than one a thread (2048 blocks);
+    right-hand sides in groups of four and a rest.  The returned maxima are
+    those of the returned X, which tol = 1e-3 leaves with the FP32 factor's
+    residual, about 1e-7 of the sums that it is the rest of (the matrices are
+    grids with 1 added to the diagonal, of condition number below 9).  A
+    residual of five products is computed to 8 u of these sums on either side:
+    4e-15 of them in all."""
+    print(f"case: refinement norms, mesh3d {mesh} x 1, nrhs {nrhs}, method {method}", flush=True)
+    G = T.mesh3d(*mesh, 1)
+    n, cp, ri, v = G.arrays()
+    A = T.from_arrays(n, cp, ri, v + (ri == np.repeat(np.arange(n), np.diff(cp))))
+    perm, inv = T.order(A, "genmmd")
+    PA = T.permute(A, perm, inv)
+    F = T.factor_symbolic(PA)
+    assert F.numeric(PA, T.FP32) == 0
+    B = np.random.default_rng(3).uniform(-1, 1, (n, nrhs))
+    X, info = F.solve_refined(PA, B, method=method, tol=1e-3, maxit=50)
+    assert info.converged
+    M = PA.to_scipy_full()
+    R = B - M @ X
+    eta = (np.abs(R).max(0) / (abs(M).sum(1).max() * np.abs(X).max(0) + np.abs(B).max(0))).max()
+    rel = (np.linalg.norm(R, axis=0) / np.linalg.norm(B, axis=0)).max()
+    noise = 4e-15 * (abs(M) @ np.abs(X) + np.abs(B)).max() / np.sqrt(np.mean(B * B, 0)).min()
+    assert rel <= 1e-4
+    assert abs(info.backward_error - eta) <= noise
+    assert abs(info.rel_residual - rel) <= noise
+    F.free()
