@@ -35,6 +35,7 @@ template <typename T> __global__ void k_gemm_tile128(const GemmTask*, const T*, 
 template <typename T> __global__ void k_gemm_short(const GemmTask*, const T*, T*, T*, const T*);
 __global__ void k_gemm_tile_bf16(const GemmTask*, const float*, float*, float*);
 template <typename T> __global__ void k_extend_add(const FrontDesc*, const EATask*, const int*, T*, T*);
+template <typename T> __global__ void k_extend_add_wave(const FrontDesc*, const EATask*, int, const EATask*, const int*, T*, T*);
 template <typename T> __global__ void k_extend_add_seq(const FrontDesc*, const EATask*, const EATask*, const int*, T*, T*);
 template <typename T> __global__ void k_solve_init(const FrontDesc*, const PanelTask*, int, const int*, const double*, int, T*, int);
 template <typename T> __global__ void k_fwd_step(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, T*, T*, int, int);
@@ -69,6 +70,11 @@ extern "C" void taucs_amd_set_profiling(int on) { g_profiling = on; }
     }                                                                                \
   } while (0)
 
+// Grouped extend-adds of at least so many parents take one wave a parent: four
+// parents a CU keep every SIMD busy.  One workgroup and one wave a parent (us):
+// 75248 parents 639 and 263, 5799 117 and 78, 3520 125 and 73, 1161 19 and 12;
+// 817 12 and 14, 386 13 and 13, 303 7 and 9.
+static const int EA_WAVE_MIN = 1024;
 struct Op {
   int kind;
   int start, count;  // range in the task array of that kind
@@ -76,7 +82,7 @@ struct Op {
   int lane = 0;      // 1: may run on the side stream (the lookahead's trailing update)
   bool nojoin = false;  // touches only the current outer panel: need not wait for the side stream
   int tile = 64;        // GEMM tile edge of the op's tasks (64 or 128)
-  bool grouped = false; // extend-add: the tasks are group heads (k_extend_add_seq)
+  bool grouped = false; // extend-add: the tasks are group heads (k_extend_add_seq, _wave)
   bool shortk = false;  // GEMM of 64-tiles whose tasks all have K <= 64 (k_gemm_short)
 };
 
@@ -673,7 +679,7 @@ static int dev_build(tamd_dev* D, const std::vector<SysView>& sys, bool dry = fa
     // extend-add of this level's fronts into their parents.  A parent whose
     // children at this level are all small (at most EA_CHUNK entries each, at
     // most EA_GROUP in all) gets one workgroup that adds them in sibling-rank
-    // order (k_extend_add_seq, one launch for all such parents); the children
+    // order (k_extend_add_seq or _wave, one launch for all such parents); the children
     // of the other parents go in one launch per sibling rank, split into
     // column chunks of about EA_CHUNK entries.  Either way a parent entry
     // receives its children's values in rank order.  (Chunk and group sizes
@@ -1367,7 +1373,11 @@ static int launch_numeric(tamd_dev* D, Emitter& E, bool bf16upd, bool prof)
         }
         break;
       case TAMD_OP_EXTEND:
-        if (op.grouped)
+        if (op.grouped && op.count >= EA_WAVE_MIN)
+          EMIT(lane, join, k_extend_add_wave<T>, dim3((op.count + 3) / 4), dim3(256),
+               (const FrontDesc*)D->d_fronts, (const EATask*)(D->d_ea + op.start), op.count,
+               (const EATask*)D->d_ea, (const int*)D->d_rel, L, U);
+        else if (op.grouped)
           EMIT(lane, join, k_extend_add_seq<T>, dim3(op.count), dim3(256),
                (const FrontDesc*)D->d_fronts, (const EATask*)(D->d_ea + op.start),
                (const EATask*)D->d_ea, (const int*)D->d_rel, L, U);

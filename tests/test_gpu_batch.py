@@ -217,3 +217,23 @@ def test_front_packing_is_bitwise_identical(prec):
             T.lib.taucs_amd_set_front_packing(1)
         assert res[0][0] == res[1][0]
         assert np.array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("precision", [T.FP64, T.FP32])
+def test_wave_extend_adds_equal_those_of_workgroups(precision):
+    """A level of thousands of small parents adds each one's children by one
+    wave, a level of few by one workgroup: the same sums in the same order.
+    Planes and boxes together (update parts of 1 to 44 rows, odd and even) have
+    such a level, each alone has not."""
+    print(f"case: batch of 20 planes and 20 boxes vs alone, precision {precision}", flush=True)
+    mats = shifted_systems(20, 56, 72, 5)
+    for q in range(20):
+        A = T.mesh3d(9 + q % 5, 10, 12)
+        mats.append(T.permute(A, *T.order(A, "genmmd")))
+    B = T.Batch(mats, precision=precision)
+    b = np.concatenate([T.random_uniform(m.n, 70 + q) for q, m in enumerate(mats)])
+    x = B.solve(b)
+    for q, m in enumerate(mats):
+        F = T.factor_llt_mf(m, precision=precision)
+        assert np.array_equal(x[B.xoff[q]:B.xoff[q + 1]], F.solve(b[B.xoff[q]:B.xoff[q + 1]])), q
+        F.free()
