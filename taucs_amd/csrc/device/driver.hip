@@ -43,6 +43,7 @@ template <typename T> __global__ void k_fwd_rect(const FrontDesc*, const PanelTa
 template <typename T> __global__ void k_fwd_rect_reduce(const FrontDesc*, const PanelTask*, const T*, T*, int);
 template <typename T> __global__ void k_bwd_cols_reduce(const FrontDesc*, const PanelTask*, const int*, const T*, T*, int, int);
 template <typename T> __global__ void k_solve_ext(const FrontDesc*, const PanelTask*, const int*, T*, int);
+template <typename T> __global__ void k_solve_ext_wave(const FrontDesc*, const PanelTask*, int, const PanelTask*, const int*, T*, int);
 template <typename T> __global__ void k_solve_ext_seq(const FrontDesc*, const PanelTask*, const PanelTask*, const int*, T*, int);
 template <typename T> __global__ void k_bwd_gather(const FrontDesc*, const PanelTask*, const int*, const double*, int, T*, int);
 template <typename T> __global__ void k_bwd_cols(const FrontDesc*, const PanelTask*, const T*, const T*, T*, int);
@@ -75,6 +76,10 @@ extern "C" void taucs_amd_set_profiling(int on) { g_profiling = on; }
 // 75248 parents 639 and 263, 5799 117 and 78, 3520 125 and 73, 1161 19 and 12;
 // 817 12 and 14, 386 13 and 13, 303 7 and 9.
 static const int EA_WAVE_MIN = 1024;
+// The same for the solve's grouped extend-adds, whose children's rows are few
+// loads a thread: 75248 parents 291 and 113, 3520 60 and 41, 2465 17 and 14; 1485
+// 19 and 21, 1161 18 and 19, 706 14 and 20.
+static const int EXT_WAVE_MIN = 2048;
 struct Op {
   int kind;
   int start, count;  // range in the task array of that kind
@@ -1683,8 +1688,12 @@ static int emit_solve(tamd_dev* D, Emitter& E, const SolveBufs& sb, int n, int n
         break;
       }
       case SV_EXTSEQ:
-        EMIT(0, true, k_solve_ext_seq<T>, grid, dim3(256), fr, tk, (const PanelTask*)D->d_sv_tasks,
-             (const int*)D->d_rel, W, nrhs);
+        if (op.count >= EXT_WAVE_MIN)
+          EMIT(0, true, k_solve_ext_wave<T>, dim3((op.count + 3) / 4), dim3(256), fr, tk, op.count,
+               (const PanelTask*)D->d_sv_tasks, (const int*)D->d_rel, W, nrhs);
+        else
+          EMIT(0, true, k_solve_ext_seq<T>, grid, dim3(256), fr, tk, (const PanelTask*)D->d_sv_tasks,
+               (const int*)D->d_rel, W, nrhs);
         break;
       case SV_BUPD:
         EMIT(0, true, k_bwd_upd<T>, grid, dim3(256), fr, tk, rows, L, (const double*)dX, ldx, Part, nrhs);

@@ -222,7 +222,8 @@ def test_front_packing_is_bitwise_identical(prec):
 @pytest.mark.parametrize("precision", [T.FP64, T.FP32])
 def test_wave_extend_adds_equal_those_of_workgroups(precision):
     """A level of thousands of small parents adds each one's children by one
-    wave, a level of few by one workgroup: the same sums in the same order.
+    wave, a level of few by one workgroup, in the factorization and in the
+    solve: the same sums in the same order.
     Planes and boxes together (update parts of 1 to 44 rows, odd and even) have
     such a level, each alone has not."""
     print(f"case: batch of 20 planes and 20 boxes vs alone, precision {precision}", flush=True)
