@@ -950,6 +950,38 @@ __device__ __forceinline__ void wave_sync_lds()
   __builtin_amdgcn_wave_barrier();
 }
 
+// A lane's column of a small front or of its inverse: the values at p = lo .. hi-1,
+// `stride` apart, N in flight and the next N loading behind their use (8, of 16
+// right-hand sides, whose sums fill the registers, 4).
+// (One at a time, a front waited for s + m round trips to memory, each for as
+// little as one fused multiply-add a lane: the backward launch of 42 thousand fronts
+// of an 80 x 72 x 64 grid, four right-hand sides, took 91 us, this way 60; of 54
+// thousand fronts of 512 planes, one right-hand side, 126 and 89.)
+template <typename T, int N> struct SmallRows {
+  const T* a;
+  int stride, lo, hi;
+  __device__ SmallRows(const T* a_, int stride_, int lo_, int hi_) : a(a_), stride(stride_), lo(lo_), hi(hi_) {}
+  // v <- the values at p .. p + N - 1 (past the end the last one: read, dropped)
+  __device__ __forceinline__ void fetch(T (&v)[N], int p) const
+  {
+#pragma unroll
+    for (int q = 0; q < N; q++) v[q] = a[(long long)min(p + q, hi - 1) * stride];
+  }
+  // use(p, value) in order; v: the first N, fetched ahead
+  template <typename F> __device__ __forceinline__ void each(T (&v)[N], F use) const
+  {
+    for (int p = lo; p < hi; p += N) {
+      T c[N];
+#pragma unroll
+      for (int q = 0; q < N; q++) c[q] = v[q];
+      if (p + N < hi) fetch(v, p + N);
+#pragma unroll
+      for (int q = 0; q < N; q++)
+        if (p + q < hi) use(p + q, c[q]);
+    }
+  }
+};
+
 // NR: right-hand sides per pass rounded up to 1, 4, 8 or 16 (compile-time, so
 // the loops over them carry no guards); columns beyond nrhs hold zeros.
 template <typename T, int NR>
@@ -960,12 +992,19 @@ __global__ __launch_bounds__(256) void k_fwd_small(const FrontDesc* __restrict__
                                                    const T* __restrict__ Inv, T* __restrict__ W,
                                                    T* __restrict__ Y, int ldy, int nrhs)
 {
+  constexpr int NB = NR <= 8 ? 8 : 4;
+  typedef SmallRows<T, NB> Rows;
   __shared__ T Ws[4][64 * NR];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ti = blockIdx.x * 4 + wv;
   if (ti >= count) return;
   const FrontDesc d = fr[tasks[ti].front];
   const int m = d.m, s = d.s;
+  const Rows iv(Inv + d.offI + min(lane, s - 1) * 64, 1, 0, s);
+  const Rows lf(L + d.offL + min(lane, m - 1), m, 0, s);
+  T ia[NB], la[NB];
+  iv.fetch(ia, 0);
+  lf.fetch(la, 0);
   T* w = W + d.offW * nrhs;
   T* ws = Ws[wv];
   const int* rw = rows + d.rows;
@@ -976,15 +1015,14 @@ __global__ __launch_bounds__(256) void k_fwd_small(const FrontDesc* __restrict__
     ws[lane + r * 64] = v[r];
   }
   wave_sync_lds();
-  const T* iv = Inv + d.offI + lane * 64;
   T y[NR];
 #pragma unroll
   for (int r = 0; r < NR; r++) y[r] = (T)0;
-  for (int p = 0; p < s; p++) {
-    const T a = (lane < s && p <= lane) ? iv[p] : (T)0;
+  iv.each(ia, [&](int p, T a) {
+    a = (lane < s && p <= lane) ? a : (T)0;
 #pragma unroll
     for (int r = 0; r < NR; r++) y[r] += a * ws[p + r * 64];
-  }
+  });
   wave_sync_lds();
   if (lane < s) {
 #pragma unroll
@@ -995,12 +1033,11 @@ __global__ __launch_bounds__(256) void k_fwd_small(const FrontDesc* __restrict__
   }
   wave_sync_lds();
   if (m == s) return;
-  const T* Lf = L + d.offL;
-  for (int p = 0; p < s; p++) {
-    const T a = (lane >= s && lane < m) ? Lf[lane + (long long)p * m] : (T)0;
+  lf.each(la, [&](int p, T a) {
+    a = (lane >= s && lane < m) ? a : (T)0;
 #pragma unroll
     for (int r = 0; r < NR; r++) v[r] -= a * ws[p + r * 64];
-  }
+  });
   if (lane >= s && lane < m) {
 #pragma unroll
     for (int r = 0; r < NR; r++)
@@ -1017,12 +1054,20 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
                                                    const T* __restrict__ Y, int ldy,
                                                    double* __restrict__ x, int ldx, int nrhs)
 {
+  constexpr int NB = NR <= 8 ? 8 : 4;
+  typedef SmallRows<T, NB> Rows;
   __shared__ T Ws[4][64 * NR];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ti = blockIdx.x * 4 + wv;
   if (ti >= count) return;
   const FrontDesc d = fr[tasks[ti].front];
   const int m = d.m, s = d.s;
+  // column `lane` of the panel's update rows and of the inverse
+  const Rows lf(L + d.offL + (long long)min(lane, s - 1) * m, 1, s, m);
+  const Rows iv(Inv + d.offI + min(lane, s - 1), 64, 0, s);
+  T la[NB], ia[NB];
+  lf.fetch(la, s);
+  iv.fetch(ia, 0);
   const int* rw = rows + d.rows;
   T* ws = Ws[wv];
   T z[NR];
@@ -1033,26 +1078,24 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
         (r < nrhs && lane >= s && lane < m) ? (T)x[rw[lane] + (long long)r * ldx] : (T)0;
   }
   wave_sync_lds();
-  const T* Lf = L + d.offL + (long long)lane * m;  // column `lane` of the panel
-  for (int i = s; i < m; i++) {
-    const T a = lane < s ? Lf[i] : (T)0;
+  lf.each(la, [&](int i, T a) {
+    a = lane < s ? a : (T)0;
 #pragma unroll
     for (int r = 0; r < NR; r++) z[r] -= a * ws[i + r * 64];
-  }
+  });
   if (lane < s) {
 #pragma unroll
     for (int r = 0; r < NR; r++) ws[lane + r * 64] = z[r];
   }
   wave_sync_lds();
-  const T* iv = Inv + d.offI + lane;  // column `lane` of the inverse: iv[p * 64]
   T xv[NR];
 #pragma unroll
   for (int r = 0; r < NR; r++) xv[r] = (T)0;
-  for (int p = 0; p < s; p++) {
-    const T a = (lane < s && p >= lane) ? iv[p * 64] : (T)0;
+  iv.each(ia, [&](int p, T a) {
+    a = (lane < s && p >= lane) ? a : (T)0;
 #pragma unroll
     for (int r = 0; r < NR; r++) xv[r] += a * ws[p + r * 64];
-  }
+  });
   if (lane < s) {
 #pragma unroll
     for (int r = 0; r < NR; r++)
