@@ -247,26 +247,30 @@ __global__ void k_solve_ext(const FrontDesc* __restrict__ fr, const PanelTask* _
   ext_row(wp + r[i], p.m, wc + i, c.m, nrhs);
 }
 
-// The same for parents whose children at this level are all small: one
-// workgroup per parent, heads[b] = {front: first task, k0: count}, the
-// children's tasks (whole update parts, nr <= blockDim) added in sibling-rank
-// order, so each parent row receives its children's values in the same order
-// as under the per-rank launches.
+// The children's updates of a level in one launch: one workgroup per parent, or
+// per piece of a wide parent's rows, heads[b] = {front: first task, k0: count}, a
+// task the rows r0 .. r0+nr-1 of a child's update part, added in sibling-rank
+// order, so each parent row receives its children's values in that order.
 template <typename T>
 __global__ void k_solve_ext_seq(const FrontDesc* __restrict__ fr, const PanelTask* __restrict__ heads,
                                 const PanelTask* __restrict__ tasks, const int* __restrict__ rel,
                                 T* __restrict__ W, int nrhs)
 {
   const PanelTask h = heads[blockIdx.x];
+  PanelTask t = tasks[h.front];
+  FrontDesc c = fr[t.front];
+  const FrontDesc p = fr[c.parent];
+  T* wp = W + p.offW * nrhs;
   for (int q = 0; q < h.k0; q++) {
     if (q > 0) __syncthreads();
-    const PanelTask t = tasks[h.front + q];
-    const FrontDesc c = fr[t.front];
-    const FrontDesc p = fr[c.parent];
-    const int* r = rel + c.rel;
-    T* wp = W + p.offW * nrhs;
-    const T* wc = W + c.offW * nrhs + c.s;
-    for (int i = threadIdx.x; i < t.nr; i += blockDim.x) ext_row(wp + r[i], p.m, wc + i, c.m, nrhs);
+    const int* r = rel + c.rel + t.r0;
+    const T* wc = W + c.offW * nrhs + c.s + t.r0;
+    const int m = c.m, nr = t.nr;
+    if (q + 1 < h.k0) {
+      t = tasks[h.front + q + 1];
+      c = fr[t.front];
+    }
+    for (int i = threadIdx.x; i < nr; i += blockDim.x) ext_row(wp + r[i], p.m, wc + i, m, nrhs);
   }
 }
 
@@ -292,8 +296,8 @@ __global__ __launch_bounds__(256) void k_solve_ext_wave(const FrontDesc* __restr
   const FrontDesc p = fr[c.parent];
   T* wp = W + p.offW * nrhs;
   for (int q = 0; q < h.k0; q++) {
-    const int* r = rel + c.rel;
-    const T* wc = W + c.offW * nrhs + c.s;
+    const int* r = rel + c.rel + t.r0;
+    const T* wc = W + c.offW * nrhs + c.s + t.r0;
     const int m = c.m, nr = t.nr;
     if (q + 1 < h.k0) {
       t = tasks[h.front + q + 1];
