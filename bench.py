@@ -604,7 +604,7 @@ def main():
         "mixed": mixed,
         "roofline": {"bound": "mfma",
                      "kernel": ("k_gemm_tile128<double>: trailing updates and SYRKs of the launches with at "
-                                "least 512 tiles of 128x128 (eight waves of 64x32, v_mfma_f64_16x16x4f64)"),
+                                "least 512 tiles of 128x128 (four waves of 64x64, v_mfma_f64_16x16x4f64)"),
                      "achieved": round(rate128 / 1e12, 3), "peak": PEAK_FP64 / 1e12,
                      "unit": "TFLOP/s", "frac": round(rate128 / PEAK_FP64, 4),
                      "avg_launch_ms": round(ms128 / max(n128, 1), 4), "launches": n128,

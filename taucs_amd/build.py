@@ -26,9 +26,8 @@ HIP_FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-Wno-unuse
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-I" + os.path.join(ROOT, "include")]
 # Per-file additions.  The factor kernels keep MFMA accumulators in
-# ordinary VGPRs: a 64x64 FP64 tile wave then needs 104 registers instead of
-# 128, so two of them leave room on a SIMD for the 288-register panel POTRF
-# wave, which must run beside the trailing update.
+# ordinary VGPRs, so that their epilogues use them without moves: the 128x128
+# FP64 tile takes 215, the 64x64 one 106 (four waves a SIMD).
 FILE_FLAGS = {"factor_kernels.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 C_FLAGS = ["-O2", "-fPIC", "-std=gnu99", "-Wall", "-Wno-unused-function",
            "-I" + os.path.join(ROOT, "include")]
