@@ -51,7 +51,7 @@ template <typename T> __global__ void k_bwd_step(const FrontDesc*, const PanelTa
 template <typename T> __global__ void k_sweep_clear(T*, double*, int, int, int, int*, int);
 template <typename T, int NSET> __global__ void k_fwd_chain(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, T*, T*, int, int*, int*, int);
 template <typename T, int NSET> __global__ void k_bwd_chain(const FrontDesc*, const PanelTask*, const int*, const T*, const T*, const T*, int, const T*, double*, int, int*, int*, int);
-template <typename T> __global__ void k_bwd_upd(const FrontDesc*, const PanelTask*, const int*, const T*, const double*, int, T*, int);
+template <typename T, int NSET> __global__ void k_bwd_upd(const FrontDesc*, const PanelTask*, const int*, const T*, const double*, int, T*, int);
 template <typename T, int NR> __global__ void k_fwd_small(const FrontDesc*, const PanelTask*, int, const int*, const T*, const T*, T*, T*, int, int);
 template <typename T, int NR> __global__ void k_bwd_small(const FrontDesc*, const PanelTask*, int, const int*, const T*, const T*, const T*, int, double*, int, int);
 }  // namespace tamd
@@ -1693,9 +1693,11 @@ static int emit_solve(tamd_dev* D, Emitter& E, const SolveBufs& sb, int n, int n
           EMIT(0, true, k_solve_ext_seq<T>, grid, dim3(256), fr, tk, (const PanelTask*)D->d_sv_tasks,
                (const int*)D->d_rel, W, nrhs);
         break;
-      case SV_BUPD:
-        EMIT(0, true, k_bwd_upd<T>, grid, dim3(256), fr, tk, rows, L, (const double*)dX, ldx, Part, nrhs);
+      case SV_BUPD: {
+        auto k = nrhs <= 4 ? k_bwd_upd<T, 1> : nrhs <= 8 ? k_bwd_upd<T, 2> : k_bwd_upd<T, 4>;
+        EMIT(0, true, k, grid, dim3(256), fr, tk, rows, L, (const double*)dX, ldx, Part, nrhs);
         break;
+      }
       case SV_BSMALL: {
         auto k = nrhs <= 1   ? k_bwd_small<T, 1>
                  : nrhs <= 4 ? k_bwd_small<T, 4>

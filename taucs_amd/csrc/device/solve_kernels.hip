@@ -467,10 +467,6 @@ __global__ __launch_bounds__(256) void k_bwd_step(const FrontDesc* __restrict__ 
 
 // (Sentinel<T>, publish: the readiness protocol, in kernels.h)
 
-// Right-hand-side blocks of the chained kernels live in LDS as 64 x 16
-// arrays [row][rhs], their rows padded against bank conflicts (YS: k_bwd_upd's).
-#define YS 17
-
 // One wave's 16 rows of a product with a 64 x 16 right-hand-side block in LDS,
 // in NSET sets of four right-hand sides (1, 2 or 4), on the MFMAs made of 4 x 4
 // blocks: FP64 4 x 4 x 4, four blocks = 16 rows, 16 cycles a set; FP32 4 x 4 x 1,
@@ -912,8 +908,10 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const FrontDesc* __restrict__
 // slots from Y in order.  x of the update rows is final (the ancestors'
 // levels wrote it) and is read through the front's row list.  MFMA as in
 // k_bwd_chain: wave w owns columns 16w..16w+15, A = L^T, B = x rows in LDS.
+// (One chain of 32 MFMAs: at 16 instead of 64 cycles each, solve of mesh3d 40^3
+// with one right-hand side 956 -> 945 us.)
 #define BU_ROWS 128
-template <typename T>
+template <typename T, int NSET>
 __global__ __launch_bounds__(256) void k_bwd_upd(const FrontDesc* __restrict__ fr,
                                                  const PanelTask* __restrict__ tasks,
                                                  const int* __restrict__ rows,
@@ -921,8 +919,8 @@ __global__ __launch_bounds__(256) void k_bwd_upd(const FrontDesc* __restrict__ f
                                                  const double* __restrict__ x, int ldx,
                                                  T* __restrict__ Part, int nrhs)
 {
-  typedef typename Mfma<T>::acc_t acc_t;
-  __shared__ T Xl[BU_ROWS * YS];
+  typedef RhsTile<T, NSET> R;
+  __shared__ alignas(16) T Xl[BU_ROWS * R::LD];
   const PanelTask t = tasks[blockIdx.x];
   const FrontDesc d = fr[t.front];
   const int m = d.m, i0 = t.k0, cnt = t.kb, c0 = t.r0, nc = t.nr;
@@ -939,21 +937,24 @@ __global__ __launch_bounds__(256) void k_bwd_upd(const FrontDesc* __restrict__ f
 #pragma unroll
   for (int k = 0; k < BU_ROWS * 16 / 256; k++) {
     const int e = tid + 256 * k, i = e & (BU_ROWS - 1), r = e / BU_ROWS;
-    Xl[i * YS + r] = (i < cnt && r < nrhs) ? (T)x[rw[i0 + i] + (long long)r * ldx] : (T)0;
+    Xl[i * R::LD + R::pos(r)] = (i < cnt && r < nrhs) ? (T)x[rw[i0 + i] + (long long)r * ldx] : (T)0;
   }
   __syncthreads();
-  acc_t D;
-#pragma unroll
-  for (int k = 0; k < 4; k++) D[k] = (T)0;
+  typename R::acc_t D0, zero;
+  R::zero(D0);
+  R::zero(zero);
   const int nst = (cnt + 3) >> 2;
 #pragma unroll
   for (int st = 0; st < BU_ROWS / 4; st++)
-    if (st < nst) D = Mfma<T>::step(a[st], Xl[(4 * st + kq) * YS + c16], D);
-  // slot stride 64 x nrhs: the columns c16 >= nrhs are not stored
+    if (st < nst) R::step(a[st], Xl + (4 * st + kq) * R::LD, lane, D0);
+  T D[NSET];
+  R::sum(D0, zero, D);
+  // slot stride 64 x nrhs: the columns c >= nrhs are not stored
   T* part = Part + (long long)blockIdx.x * (64LL * nrhs);
-  if (c16 < nrhs) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) part[16 * wv + Mfma<T>::drow(lane, k) + c16 * 64] = D[k];
+  for (int k = 0; k < NSET; k++) {
+    const int c = R::col(lane, k);
+    if (c < nrhs) part[16 * wv + R::row(lane, k) + c * 64] = D[k];
   }
 }
 
@@ -1131,7 +1132,9 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
                                                 const T*, const T*, T*, T*, int, int*, int*, int); \
   template __global__ void k_bwd_chain<T, NSET>(const FrontDesc*, const PanelTask*, const int*, \
                                                 const T*, const T*, const T*, int, const T*,    \
-                                                double*, int, int*, int*, int);
+                                                double*, int, int*, int*, int);                          \
+  template __global__ void k_bwd_upd<T, NSET>(const FrontDesc*, const PanelTask*, const int*,   \
+                                              const T*, const double*, int, T*, int);
 #define TAMD_SINST(T)                                                                           \
   template __global__ void k_solve_init<T>(const FrontDesc*, const PanelTask*, int, const int*,  \
                                            const double*, int, T*, int);                        \
@@ -1155,8 +1158,6 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
                                          const T*, const T*, T*, int, double*, int, int);       \
   template __global__ void k_sweep_clear<T>(T*, double*, int, int, int, int*, int);           \
   CHAIN_INST(T, 1) CHAIN_INST(T, 2) CHAIN_INST(T, 4)                                            \
-  template __global__ void k_bwd_upd<T>(const FrontDesc*, const PanelTask*, const int*, const T*, \
-                                        const double*, int, T*, int);                          \
   SMALL_INST(T, 1) SMALL_INST(T, 4) SMALL_INST(T, 8) SMALL_INST(T, 16)
 TAMD_SINST(double)
 TAMD_SINST(float)
