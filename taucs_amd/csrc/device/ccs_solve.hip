@@ -287,14 +287,13 @@ extern "C" int taucs_ccs_solve_llt(void* vL, void* vx, void* vb)
     int* w = (int*)buf[8];
     const long long fill = 2LL * n;
     unsigned g = (unsigned)std::min<long long>((fill + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_ccs_fill, dim3(g), dim3(256), 0, 0, y, fill, w, 4);
-    hipLaunchKernelGGL(k_ccs_fwd, dim3(n), dim3(64), 0, 0, n, (const int*)buf[3],
-                       (const int*)buf[4], (const double*)buf[5], (const double*)buf[6], y, w,
-                       w + 2);
-    hipLaunchKernelGGL(k_ccs_bwd, dim3(n), dim3(64), 0, 0, n, (const int*)buf[0],
-                       (const int*)buf[1], (const double*)buf[2], (const double*)y, y + n, w + 1,
-                       w + 2);
-    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) rc = -1;
+    if (launch(k_ccs_fill, dim3(g), dim3(256), 0, y, fill, w, 4) != hipSuccess
+        || launch(k_ccs_fwd, dim3(n), dim3(64), 0, n, (const int*)buf[3], (const int*)buf[4],
+                  (const double*)buf[5], (const double*)buf[6], y, w, w + 2) != hipSuccess
+        || launch(k_ccs_bwd, dim3(n), dim3(64), 0, n, (const int*)buf[0], (const int*)buf[1],
+                  (const double*)buf[2], (const double*)y, y + n, w + 1, w + 2) != hipSuccess
+        || hipDeviceSynchronize() != hipSuccess)
+      rc = -1;
     if (rc == 0) rc = taucs_amd_memcpy_d2h(words, w, ib * 4) || taucs_amd_memcpy_d2h(x, y + n, db * n);
     if (rc == 0 && words[2]) {
       taucs_printf((char*)"taucs_ccs_solve_llt: a sweep timed out waiting for a value\n");

@@ -1466,7 +1466,6 @@ static int run_numeric(tamd_dev* D, bool bf16upd)
     HIPCHECK(hipGraphLaunch(D->num_graph, st));
     D->timing.launches = D->num_graph_launches;
   }
-  HIPCHECK(hipGetLastError());
   if (prof) {
     float ms = 0;
     HIPCHECK(hipEventRecord(e1, st));
@@ -1740,7 +1739,6 @@ static int run_solve(tamd_factor* F, int nrhs, double* dX, int ldx, const double
   if (!g_graphs) {
     Emitter E = eager_emitter(D);
     if (emit_solve<T>(D, E, sb, n, nrhs, dX, ldx, dB, ldb) != 0) return -1;
-    HIPCHECK(hipGetLastError());
     return 0;
   }
   for (auto& g : D->sv)
@@ -1858,7 +1856,6 @@ extern "C" int tamd_dev_solve_eager(tamd_factor* F, void* W, void* Y, void* Part
                      ? emit_solve<double>(D, E, sb, F->n, nr, dX, ldx, dB, ldb)
                      : emit_solve<float>(D, E, sb, F->n, nr, dX, ldx, dB, ldb);
   if (rc != 0) return -1;
-  HIPCHECK(hipGetLastError());
   return 0;
 }
 
@@ -1933,9 +1930,7 @@ extern "C" int taucs_amd_factor_digest(void* vL, unsigned long long* digest)
   int rc = 0;
   if (hipMemsetAsync(d_out, 0, sizeof(unsigned long long), D->stream) != hipSuccess) rc = -1;
   if (!rc) {
-    hipLaunchKernelGGL(k_digest, dim3(2048), dim3(256), 0, D->stream, (const unsigned int*)D->L, nw,
-                       d_out);
-    if (hipGetLastError() != hipSuccess
+    if (launch(k_digest, dim3(2048), dim3(256), D->stream, (const unsigned int*)D->L, nw, d_out) != hipSuccess
         || hipMemcpyAsync(digest, d_out, sizeof(unsigned long long), hipMemcpyDeviceToHost, D->stream)
                != hipSuccess
         || hipStreamSynchronize(D->stream) != hipSuccess)

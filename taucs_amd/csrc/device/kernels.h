@@ -15,6 +15,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <tuple>
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
@@ -154,4 +155,20 @@ __device__ __forceinline__ T await_value(const T* p, int* err)
     v = __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   return __builtin_bit_cast(T, v);
+}
+
+// ---- launches ---------------------------------------------------------------
+// Launches k; the launch's own status.  (hipGetLastError gives the thread's last
+// error, which may be of an earlier call, of this library or of the program: an
+// allocation that was refused and dealt with, say.)
+template <typename... P, typename... A>
+static inline hipError_t launch(void (*k)(P...), dim3 grid, dim3 block, hipStream_t st, A... a)
+{
+  std::tuple<P...> v(a...);
+  return std::apply(
+      [&](P&... p) {
+        void* args[] = {(void*)&p...};
+        return hipLaunchKernel((const void*)k, grid, block, args, 0, st);
+      },
+      v);
 }

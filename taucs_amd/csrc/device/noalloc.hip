@@ -18,6 +18,7 @@
 
 #include <mutex>
 
+#include "kernels.h"
 #include "../host/internal.h"
 
 extern "C" int tamd_dev_solve_dims(tamd_factor* F, long long* W_per_rhs, long long* part_slots,
@@ -127,8 +128,7 @@ extern "C" int taucs_amd_supernodal_solve_many_device_noalloc(void* vL, int nrhs
     const long long nw = r0 == 0 ? sync_n + 1 : sync_n;
     if (nw > 0) {
       const unsigned blocks = (unsigned)(nw < 1024 * 256 ? (nw + 255) / 256 : 1024);
-      hipLaunchKernelGGL(k_clear_words, dim3(blocks), dim3(256), 0, st, sync, nw);
-      if (hipGetLastError() != hipSuccess) return -1;
+      if (launch(k_clear_words, dim3(blocks), dim3(256), st, sync, nw) != hipSuccess) return -1;
     }
     if (tamd_dev_solve_eager(F, W, Y, Part, sync, nr, dX + (size_t)r0 * ldx, ldx,
                              dB + (size_t)r0 * ldb, ldb) != 0)

@@ -422,14 +422,12 @@ static int residual_and_error(hipStream_t st, RefineCtx* c, const double* x, con
   const int n = c->n, nblk = row_blocks(n);
   double* const anorm = c->norms + NQ * (size_t)c->cap;
   if (c->anorm_stale) {  // |A|_inf = max row sum of |a_ij|
-    hipLaunchKernelGGL(k_csr_absrow, dim3(nblk), dim3(256), 0, st, n, c->rp, c->v, c->partial);
-    hipLaunchKernelGGL(k_norms_final, dim3(1), dim3(256), 0, st, nblk, c->partial, 1, anorm);
+    HIPOK(launch(k_csr_absrow, dim3(nblk), dim3(256), st, n, c->rp, c->v, c->partial));
+    HIPOK(launch(k_norms_final, dim3(1), dim3(256), st, nblk, c->partial, 1, anorm));
   }
-  hipLaunchKernelGGL(k_csr_residual<false>, dim3(nblk, (nrhs + 3) / 4), dim3(256), 0, st, n, c->rp, c->ci,
-                     c->v, x, b, r, nrhs, c->partial);
-  hipLaunchKernelGGL(k_norms_final, dim3(NQ * nrhs), dim3(256), 0, st, nblk, c->partial, 3 * nrhs,
-                     c->norms);
-  HIPOK(hipGetLastError());
+  HIPOK(launch(k_csr_residual<false>, dim3(nblk, (nrhs + 3) / 4), dim3(256), st, n, c->rp, c->ci, c->v,
+               x, b, r, nrhs, c->partial));
+  HIPOK(launch(k_norms_final, dim3(NQ * nrhs), dim3(256), st, nblk, c->partial, 3 * nrhs, c->norms));
   HIPOK(hipStreamSynchronize(st));
   if (c->anorm_stale) c->anorm_inf = *anorm;
   c->anorm_stale = false;

@@ -1,0 +1,68 @@
+"""Calls beside failures that are not their own, and refinement after its own."""
+import numpy as np
+import pytest
+
+import taucs_amd as T
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(side):
+    A = T.mesh3d(side)
+    perm, inv = T.order(A, "genmmd")
+    return T.permute(A, perm, inv)
+
+
+def test_calls_after_a_refused_allocation():
+    """An allocation that the device refused, and that the program has dealt
+    with, is no failure of the calls that follow: factorization, digest, solves
+    (host, device and allocation-free; graphs and eager launches), refinement
+    and the CCS solve give the bits that they gave before it."""
+    PA = _system(9)
+    b = np.random.default_rng(2).uniform(-1, 1, (PA.n, 3))
+
+    def calls():
+        out = []
+        for prec in (T.FP64, T.FP32):
+            print(f"case: calls beside a refused allocation, precision {prec}", flush=True)
+            yield
+            F = T.factor_llt_mf(PA, precision=prec)
+            yield
+            out.append(F.digest())
+            yield
+            out.append(F.solve(b))
+            for method in (0, 1):
+                yield
+                x, info = F.solve_refined(PA, b, method=method)
+                assert info.converged
+                out.append(x)
+            dB, dX = T.DeviceArray(b), T.DeviceArray(np.zeros_like(b))
+            yield
+            rc = T.lib.taucs_amd_supernodal_solve_many_device_noalloc(F.h, 3, dX.ptr, PA.n, dB.ptr, PA.n)
+            assert rc == 0
+            out.append(dX.get())
+            try:
+                T.lib.taucs_amd_set_graphs(0)
+                yield
+                assert F.numeric(PA, prec) == 0
+                yield
+                F.solve_device(dX.ptr, dB.ptr, PA.n, 3)
+            finally:
+                T.lib.taucs_amd_set_graphs(1)
+            out.append(dX.get())
+            if prec == T.FP64:
+                L = F.to_ccs()
+                yield
+                out.append(L.solve_llt(b[:, 0]))
+            dB.free()
+            dX.free()
+            F.free()
+        results.append(out)
+
+    results = []
+    for refused in (False, True):
+        for _ in calls():
+            if refused:
+                assert not T.lib.taucs_amd_device_malloc(1 << 46)  # 64 TiB
+    for x0, x1 in zip(*results):
+        assert np.array_equal(x0, x1)
