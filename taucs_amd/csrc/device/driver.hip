@@ -264,6 +264,24 @@ static void free_ptr(void* p)
   }
 }
 
+// Pinned host memory, with the same induced failures and message; it takes no HBM
+// and is not in the ledger.
+extern "C" int tamd_pinned_malloc(void** p, size_t bytes)
+{
+  const bool induced = tamd_alloc_should_fail();
+  const hipError_t e = induced ? hipErrorOutOfMemory : hipHostMalloc(p, bytes, 0);
+  if (e == hipSuccess) return 0;
+  *p = nullptr;
+  taucs_printf((char*)"taucs_amd: hipHostMalloc(%zu) failed: %s\n", bytes,
+               induced ? "induced" : hipGetErrorString(e));
+  return -1;
+}
+
+extern "C" void tamd_pinned_free(void* p)
+{
+  if (p) (void)hipHostFree(p);
+}
+
 extern "C" int tamd_dev_malloc(void** p, size_t bytes) { return dev_malloc(p, bytes); }
 extern "C" void tamd_dev_free_ptr(void* p) { free_ptr(p); }
 

@@ -256,6 +256,8 @@ static std::mutex g_ctx_mu;
 
 extern "C" int tamd_dev_malloc(void** p, size_t bytes);
 extern "C" void tamd_dev_free_ptr(void* p);
+extern "C" int tamd_pinned_malloc(void** p, size_t bytes);
+extern "C" void tamd_pinned_free(void* p);
 
 static void ctx_free(RefineCtx* c)
 {
@@ -263,7 +265,7 @@ static void ctx_free(RefineCtx* c)
   void* ps[] = {c->rp, c->ci, c->src, c->v, c->avals, c->r, c->z, c->p, c->q, c->x, c->b, c->partial,
                 c->mask, c->rz, c->scal, c->done};
   for (void* p : ps) tamd_dev_free_ptr(p);
-  if (c->norms) (void)hipHostFree(c->norms);
+  tamd_pinned_free(c->norms);
   delete c;
 }
 
@@ -398,12 +400,9 @@ static RefineCtx* get_ctx(tamd_factor* F, const taucs_ccs_matrix* A, int nrhs, b
       *e.p = nullptr;
       if (dmalloc(e.p, e.bytes)) return nullptr;
     }
-    if (c->norms) (void)hipHostFree(c->norms);
+    tamd_pinned_free(c->norms);
     c->norms = nullptr;
-    if (hipHostMalloc((void**)&c->norms, sizeof(double) * (NQ * (size_t)nrhs + 1), 0) != hipSuccess) {
-      c->norms = nullptr;
-      return nullptr;
-    }
+    if (tamd_pinned_malloc((void**)&c->norms, sizeof(double) * (NQ * (size_t)nrhs + 1))) return nullptr;
     c->cap = nrhs;
   }
   return c;
