@@ -243,6 +243,14 @@ int  taucs_amd_get_op_profile(void* L, int cap, int* kind, int* level, int* coun
    updates, k_gemm_short).  Returns the op count, or -1 without a device
    schedule.  No counterpart in the reference (inspection). */
 int  taucs_amd_get_op_tiles(void* L, int cap, int* tile, int* shortk);
+/* The extend-add launches that add several children to each parent, in launch
+   order, of the factorization (solve = 0) or of the chained solve (solve = 1):
+   the parents (or pieces of wide parents) of each, and how many of these one
+   wave each takes, the others a workgroup each.  Returns the number of such
+   launches, or -1 without a device schedule.  No counterpart in the reference
+   (inspection). */
+int  taucs_amd_get_extend_adds(void* L, int solve, int cap, int* parents, int* waves);
+int  taucs_amd_batch_get_extend_adds(void* B, int solve, int cap, int* parents, int* waves);
 
 #ifdef __cplusplus
 }

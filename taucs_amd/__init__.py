@@ -131,6 +131,8 @@ _sigs = {
                                            C.c_void_p, C.c_void_p]),
     "taucs_amd_get_op_profile": (C.c_int, [C.c_void_p, C.c_int] + [C.c_void_p] * 6),
     "taucs_amd_get_op_tiles": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
+    "taucs_amd_get_extend_adds": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p]),
+    "taucs_amd_batch_get_extend_adds": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p]),
     "taucs_amd_batch_factor_llt_mf": (C.c_void_p, [C.c_void_p, C.c_void_p, C.c_int]),
     "taucs_amd_batch_numeric": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int]),
     "taucs_amd_batch_solve": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int]),
@@ -337,6 +339,15 @@ def _refine_method(method, factored, stop_relres):
         (REFINE_STOP_RELRES if stop_relres else 0)
 
 
+def _extend_adds(get, h, solve):
+    n = get(h, int(solve), 0, None, None)
+    if n < 0:
+        raise RuntimeError("no device schedule")
+    parents, waves = np.zeros(n, dtype=np.int32), np.zeros(n, dtype=np.int32)
+    get(h, int(solve), n, _dptr(parents), _dptr(waves))
+    return {"parents": parents, "waves": waves}
+
+
 class Factor:
     """Owner of an opaque device-resident supernodal factor."""
 
@@ -488,6 +499,10 @@ class Factor:
         lib.taucs_amd_get_op_tiles(self.h, n, _dptr(tile), _dptr(shortk))
         return {"kind": k, "level": lv, "count": c, "flops": f, "bytes": b, "ms": ms, "tile": tile,
                 "shortk": shortk}
+
+    def extend_adds(self, solve=False):
+        """Parents of each grouped extend-add launch, and how many of them one wave each takes."""
+        return _extend_adds(lib.taucs_amd_get_extend_adds, self.h, solve)
 
     def free(self):
         if self.h:
@@ -654,6 +669,10 @@ class Batch:
         t = NumericTiming()
         lib.taucs_amd_batch_get_timing(self.h, C.byref(t))
         return t
+
+    def extend_adds(self, solve=False):
+        """Factor.extend_adds of the batch's schedule."""
+        return _extend_adds(lib.taucs_amd_batch_get_extend_adds, self.h, solve)
 
     def free(self):
         if self.h:

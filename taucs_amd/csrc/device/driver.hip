@@ -43,7 +43,7 @@ template <typename T> __global__ void k_fwd_rect(const FrontDesc*, const PanelTa
 template <typename T> __global__ void k_fwd_rect_reduce(const FrontDesc*, const PanelTask*, const T*, T*, int);
 template <typename T> __global__ void k_bwd_cols_reduce(const FrontDesc*, const PanelTask*, const int*, const T*, T*, int, int);
 template <typename T> __global__ void k_solve_ext(const FrontDesc*, const PanelTask*, const int*, T*, int);
-template <typename T> __global__ void k_solve_ext_wave(const FrontDesc*, const PanelTask*, int, const PanelTask*, const int*, T*, int);
+template <typename T> __global__ void k_solve_ext_wave(const FrontDesc*, const PanelTask*, int, int, const PanelTask*, const int*, T*, int);
 template <typename T> __global__ void k_solve_ext_seq(const FrontDesc*, const PanelTask*, const PanelTask*, const int*, T*, int);
 template <typename T> __global__ void k_bwd_gather(const FrontDesc*, const PanelTask*, const int*, const double*, int, T*, int);
 template <typename T> __global__ void k_bwd_cols(const FrontDesc*, const PanelTask*, const T*, const T*, T*, int);
@@ -80,6 +80,17 @@ static const int EA_WAVE_MIN = 1024;
 // loads a thread: 75248 parents 291 and 113, 3520 60 and 41, 2465 17 and 14; 1485
 // 19 and 21, 1161 18 and 19, 706 14 and 20.
 static const int EXT_WAVE_MIN = 2048;
+// A wave takes a child's rows 64 at a time, about 0.7 us each further 64 with one
+// right-hand side and 1.5 with 16, where a workgroup takes 256 at once.  A parent
+// for which that is more than so many times in all keeps a workgroup of the launch
+// to itself: the launch would wait for its wave alone.  (2600 parents of eight
+// children of 16 rows and one of 100 children of 250, solve with 1 and 16 right-hand
+// sides: all by workgroups 509 and 1147 us, all by waves 698 and 1559, this way
+// 477 and 1096; one of 100 children of 400 529 and 1158, 727 and 1630, 500 and 1113.
+// 3000 alike of eight children of 128 rows, which stay with the waves: workgroups
+// 1607 and 2998, waves 1590 and 3018; of 200 rows, which do not: 2416 and 4540,
+// 2413 and 4574.)
+static const int EXT_WAVE_MORE = 8;
 struct Op {
   int kind;
   int start, count;  // range in the task array of that kind
@@ -89,7 +100,11 @@ struct Op {
   int tile = 64;        // GEMM tile edge of the op's tasks (64 or 128)
   bool grouped = false; // extend-add: the tasks are group heads (k_extend_add_seq, _wave)
   bool shortk = false;  // GEMM of 64-tiles whose tasks all have K <= 64 (k_gemm_short)
+  int wide = 0;         // solve extend-add by waves: the first heads, a workgroup each
 };
+// how many of an extend-add launch's parents one wave each takes
+static int ea_waves(const Op& op) { return op.grouped && op.count >= EA_WAVE_MIN ? op.count : 0; }
+static int ext_waves(const Op& op) { return op.count - op.wide >= EXT_WAVE_MIN ? op.count - op.wide : 0; }
 
 // solve op kinds
 enum { SV_INIT, SV_FSTEP, SV_FRECT, SV_FRED, SV_EXT, SV_GATHER, SV_BCOLS, SV_BRED, SV_BSTEP,
@@ -934,12 +949,22 @@ static int dev_build(tamd_dev* D, const std::vector<SysView>& sys, bool dry = fa
           if ((int)body.size() > first) heads.push_back({first, (int)body.size() - first, 0, 0, 0});
         }
       }
+      // heads that a wave would be long over first (EXT_WAVE_MORE)
+      auto long_wave = [&](const PanelTask& h) {
+        int more = 0;
+        for (int q = 0; q < h.k0; q++) more += (body[h.front + q].nr - 1) / 64;
+        return more > EXT_WAVE_MORE;
+      };
+      int wide = 0;
+      if ((int)heads.size() >= EXT_WAVE_MIN)
+        wide = (int)(std::stable_partition(heads.begin(), heads.end(), long_wave) - heads.begin());
       if (!heads.empty()) {
         t0 = svt.size();
         const int bb = (int)(t0 + heads.size());
         for (PanelTask& h : heads) h.front += bb;  // heads index the bodies in the same array
         svt.insert(svt.end(), heads.begin(), heads.end());
         push_chain(SV_EXTSEQ, t0, l, false);
+        D->sv_chain_ops.back().wide = wide;
         svt.insert(svt.end(), body.begin(), body.end());
       }
     }
@@ -1394,7 +1419,7 @@ static int launch_numeric(tamd_dev* D, Emitter& E, bool bf16upd, bool prof)
         }
         break;
       case TAMD_OP_EXTEND:
-        if (op.grouped && op.count >= EA_WAVE_MIN)
+        if (ea_waves(op) > 0)
           EMIT(lane, join, k_extend_add_wave<T>, dim3((op.count + 3) / 4), dim3(256),
                (const FrontDesc*)D->d_fronts, (const EATask*)(D->d_ea + op.start), op.count,
                (const EATask*)D->d_ea, (const int*)D->d_rel, L, U);
@@ -1604,6 +1629,22 @@ extern "C" int taucs_amd_get_op_tiles(void* vL, int cap, int* tile, int* shortk)
   return n;
 }
 
+extern "C" int taucs_amd_get_extend_adds(void* vL, int solve, int cap, int* parents, int* waves)
+{
+  tamd_factor* F = (tamd_factor*)vL;
+  if (!F || !F->dev) return -1;
+  int n = 0;
+  for (const Op& op : solve ? F->dev->sv_chain_ops : F->dev->ops) {
+    if (solve ? op.kind != SV_EXTSEQ : !(op.kind == TAMD_OP_EXTEND && op.grouped)) continue;
+    if (n < cap) {
+      if (parents) parents[n] = op.count;
+      if (waves) waves[n] = solve ? ext_waves(op) : ea_waves(op);
+    }
+    n++;
+  }
+  return n;
+}
+
 extern "C" int taucs_amd_factor_fp64_fallbacks(void* vL)
 {
   tamd_factor* F = (tamd_factor*)vL;
@@ -1703,9 +1744,9 @@ static int emit_solve(tamd_dev* D, Emitter& E, const SolveBufs& sb, int n, int n
         break;
       }
       case SV_EXTSEQ:
-        if (op.count >= EXT_WAVE_MIN)
-          EMIT(0, true, k_solve_ext_wave<T>, dim3((op.count + 3) / 4), dim3(256), fr, tk, op.count,
-               (const PanelTask*)D->d_sv_tasks, (const int*)D->d_rel, W, nrhs);
+        if (ext_waves(op) > 0)
+          EMIT(0, true, k_solve_ext_wave<T>, dim3(op.wide + (op.count - op.wide + 3) / 4), dim3(256), fr, tk,
+               op.wide, op.count, (const PanelTask*)D->d_sv_tasks, (const int*)D->d_rel, W, nrhs);
         else
           EMIT(0, true, k_solve_ext_seq<T>, grid, dim3(256), fr, tk, (const PanelTask*)D->d_sv_tasks,
                (const int*)D->d_rel, W, nrhs);

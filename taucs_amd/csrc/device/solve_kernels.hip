@@ -251,18 +251,19 @@ __global__ void k_solve_ext(const FrontDesc* __restrict__ fr, const PanelTask* _
 // per piece of a wide parent's rows, heads[b] = {front: first task, k0: count}, a
 // task the rows r0 .. r0+nr-1 of a child's update part, added in sibling-rank
 // order, so each parent row receives its children's values in that order.
-template <typename T>
-__global__ void k_solve_ext_seq(const FrontDesc* __restrict__ fr, const PanelTask* __restrict__ heads,
-                                const PanelTask* __restrict__ tasks, const int* __restrict__ rel,
-                                T* __restrict__ W, int nrhs)
+// By a workgroup, or (WAVE) by one wave, whose memory operations are performed in
+// order: no barrier between children.
+template <typename T, bool WAVE>
+__device__ __forceinline__ void ext_head(const FrontDesc* __restrict__ fr, const PanelTask h,
+                                         const PanelTask* __restrict__ tasks, const int* __restrict__ rel,
+                                         T* W, int nrhs)
 {
-  const PanelTask h = heads[blockIdx.x];
   PanelTask t = tasks[h.front];
   FrontDesc c = fr[t.front];
   const FrontDesc p = fr[c.parent];
   T* wp = W + p.offW * nrhs;
   for (int q = 0; q < h.k0; q++) {
-    if (q > 0) __syncthreads();
+    if (!WAVE && q > 0) __syncthreads();
     const int* r = rel + c.rel + t.r0;
     const T* wc = W + c.offW * nrhs + c.s + t.r0;
     const int m = c.m, nr = t.nr;
@@ -270,43 +271,44 @@ __global__ void k_solve_ext_seq(const FrontDesc* __restrict__ fr, const PanelTas
       t = tasks[h.front + q + 1];
       c = fr[t.front];
     }
-    for (int i = threadIdx.x; i < nr; i += blockDim.x) ext_row(wp + r[i], p.m, wc + i, m, nrhs);
+    for (int i = WAVE ? threadIdx.x & 63 : threadIdx.x; i < nr; i += WAVE ? 64 : 256)
+      ext_row(wp + r[i], p.m, wc + i, m, nrhs);
+    if (WAVE) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_solve_ext_seq(const FrontDesc* __restrict__ fr,
+                                                       const PanelTask* __restrict__ heads,
+                                                       const PanelTask* __restrict__ tasks,
+                                                       const int* __restrict__ rel, T* W, int nrhs)
+{
+  ext_head<T, false>(fr, heads[blockIdx.x], tasks, rel, W, nrhs);
 }
 
 // The same with one parent per wave, four to a workgroup, for launches of so many
 // parents that they fill the chip: children of a few rows leave most of a
 // workgroup's threads idle, and a child's descriptors, places and values are a
-// chain of loads, so that what bounds a launch is the parents in flight.  A wave's
-// memory operations are performed in order: no barrier between children.
+// chain of loads, so that what bounds a launch is the parents in flight.
 // 512 grids of 16 to 128 points a side, 75 thousand parents in a launch, one
-// right-hand side: 291 -> 113 us.
+// right-hand side: 291 -> 113 us.  The first `wide` parents, which would keep a wave
+// long, have a workgroup each.
 template <typename T>
 __global__ __launch_bounds__(256) void k_solve_ext_wave(const FrontDesc* __restrict__ fr,
-                                                        const PanelTask* __restrict__ heads, int nheads,
-                                                        const PanelTask* __restrict__ tasks,
+                                                        const PanelTask* __restrict__ heads, int wide,
+                                                        int nheads, const PanelTask* __restrict__ tasks,
                                                         const int* __restrict__ rel, T* W, int nrhs)
 {
-  const int lane = threadIdx.x & 63;
-  const int hd = 4 * blockIdx.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (hd >= nheads) return;
-  const PanelTask h = heads[hd];
-  PanelTask t = tasks[h.front];
-  FrontDesc c = fr[t.front];
-  const FrontDesc p = fr[c.parent];
-  T* wp = W + p.offW * nrhs;
-  for (int q = 0; q < h.k0; q++) {
-    const int* r = rel + c.rel + t.r0;
-    const T* wc = W + c.offW * nrhs + c.s + t.r0;
-    const int m = c.m, nr = t.nr;
-    if (q + 1 < h.k0) {
-      t = tasks[h.front + q + 1];
-      c = fr[t.front];
-    }
-    for (int i = lane; i < nr; i += 64) ext_row(wp + r[i], p.m, wc + i, m, nrhs);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+  const int b = blockIdx.x;
+  if (b < wide) {
+    ext_head<T, false>(fr, heads[b], tasks, rel, W, nrhs);
+    return;
   }
+  const int hd = wide + 4 * (b - wide) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (hd < nheads) ext_head<T, true>(fr, heads[hd], tasks, rel, W, nrhs);
 }
 
 // Backward: W_f[s + i] <- x(update row i) for rows r0..r0+nr-1 of the update part.
@@ -1148,7 +1150,7 @@ __global__ __launch_bounds__(256) void k_bwd_small(const FrontDesc* __restrict__
   template __global__ void k_solve_ext<T>(const FrontDesc*, const PanelTask*, const int*, T*, int); \
   template __global__ void k_solve_ext_seq<T>(const FrontDesc*, const PanelTask*, const PanelTask*, \
                                               const int*, T*, int);                             \
-  template __global__ void k_solve_ext_wave<T>(const FrontDesc*, const PanelTask*, int,          \
+  template __global__ void k_solve_ext_wave<T>(const FrontDesc*, const PanelTask*, int, int,     \
                                                const PanelTask*, const int*, T*, int);          \
   template __global__ void k_bwd_gather<T>(const FrontDesc*, const PanelTask*, const int*,        \
                                            const double*, int, T*, int);                        \

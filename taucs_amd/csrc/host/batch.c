@@ -196,6 +196,13 @@ int taucs_amd_batch_get_timing(void* vB, taucs_amd_numeric_timing* t)
   return taucs_amd_get_numeric_timing(&B->all, t);
 }
 
+int taucs_amd_batch_get_extend_adds(void* vB, int solve, int cap, int* parents, int* waves)
+{
+  tamd_batch* B = (tamd_batch*)vB;
+  if (!B) return -1;
+  return taucs_amd_get_extend_adds(&B->all, solve, cap, parents, waves);
+}
+
 /* The schedule autotuner (taucs_amd_autotune) for a batch: all systems share
    one schedule, so one schedule shape is chosen for the whole batch. */
 int taucs_amd_batch_autotune(void* vB, const int* cand_w, const int* cand_tile, int ncand, int reps,

@@ -238,3 +238,54 @@ def test_wave_extend_adds_equal_those_of_workgroups(precision):
         F = T.factor_llt_mf(m, precision=precision)
         assert np.array_equal(x[B.xoff[q]:B.xoff[q + 1]], F.solve(b[B.xoff[q]:B.xoff[q + 1]])), q
         F.free()
+
+
+def bordered(leaves, s, w, seed):
+    """`leaves` dense s x s blocks, each coupled to all of a dense border of w
+    unknowns: as many fronts with s columns and w update rows, children of the
+    border's (the blocks' fill is too large for the relaxed amalgamation).  Strongly
+    diagonally dominant."""
+    rng = np.random.default_rng(seed)
+    n = leaves * s + w
+    cp, ri, v = [0], [], []
+    for j in range(n):
+        end = (j // s + 1) * s if j < leaves * s else n
+        rows = np.concatenate([np.arange(j, end), np.arange(max(end, leaves * s), n)])
+        x = rng.uniform(-1, 1, len(rows)) / 64
+        x[0] = 8 + n / 32
+        ri.append(rows)
+        v.append(x)
+        cp.append(cp[-1] + len(rows))
+    A = T.from_arrays(n, np.array(cp), np.concatenate(ri), np.concatenate(v))
+    return T.permute(A, *T.order(A, "identity"))
+
+
+@pytest.mark.parametrize("precision", [T.FP64, T.FP32])
+def test_levels_of_small_and_wide_parents(precision):
+    """A level of 2100 parents with two children of 4 rows, by waves, and beside
+    them: in the factorization parents of children of up to 44 rows (990 entries,
+    two passes of a wave) by waves too; in the solve one of children of 100 rows
+    (two passes), one of 250 rows, a workgroup's, and one of 600 rows, cut into
+    three pieces, of which the last goes to a wave.  The bits of the systems
+    factored and solved alone, where no level takes waves."""
+    small = [bordered(2, 16, 4, q) for q in range(4)]
+    mid = [bordered(8, 30, w, w) for w in (1, 2, 31, 32, 33, 43, 44)]
+    wide = [bordered(4, 70, 100, 11), bordered(12, 40, 250, 12), bordered(6, 60, 600, 13)]
+    mats = wide + mid + small * 525
+    kinds = wide + mid + small
+    print(f"case: batch of {len(mats)} bordered systems, precision {precision}", flush=True)
+    B = T.Batch(mats, precision=precision)
+    ea, ext = B.extend_adds(), B.extend_adds(solve=True)
+    assert ea["waves"][0] == ea["parents"][0] == 2100 + len(mid)
+    assert ext["parents"][0] == 2100 + len(mid) + 1 + 1 + 3
+    assert ext["waves"][0] == 2100 + len(mid) + 1 + 1
+    for nrhs in (1, 9):
+        b = np.random.default_rng(nrhs).uniform(-1, 1, (int(B.xoff[-1]), nrhs))
+        x = B.solve(b)
+        for q, m in enumerate(kinds):
+            F = T.factor_llt_mf(m, precision=precision)
+            assert F.extend_adds()["waves"].sum() == F.extend_adds(solve=True)["waves"].sum() == 0
+            at = slice(B.xoff[q], B.xoff[q + 1])
+            assert np.array_equal(x[at], F.solve(b[at])), (q, nrhs)
+            F.free()
+    B.free()
