@@ -347,3 +347,54 @@ def test_refinement_norms_at_block_edges(method, mesh, nrhs):
     assert abs(info.backward_error - eta) <= noise
     assert abs(info.rel_residual - rel) <= noise
     F.free()
+
+
+@pytest.mark.parametrize("chained", [True, False])
+@pytest.mark.parametrize("precision,real", [(T.FP64, np.float64), (T.FP32, np.float32)])
+def test_extend_adds_of_a_wide_parent_in_order(chained, precision, real):
+    """200 leaves of one column, each with some 420 of the 600 rows of one parent:
+    the chained solve cuts the parent's rows into three pieces, the other goes by
+    launches of a sibling rank.  Every product is exact here: entries of a leaf's
+    column are 1 and +-1/4, and the parent's Schur complement is the identity (sums
+    of at most 200 sixteenths).  So the parent's x is b with the leaves' shares
+    subtracted one after the other in the order of the child list, to the last bit."""
+    print(f"case: a wide parent's extend-adds in order, precision {precision}, chained {chained}", flush=True)
+    rng = np.random.default_rng(7)
+    nl, w, nrhs = 200, 600, 3
+    V = rng.choice([-0.25, 0.0, 0.25], (w, nl), p=[0.35, 0.3, 0.35])
+    V[0] = 0.25  # all leaves hang on the parent's first row
+    S = np.eye(w) + V @ V.T
+    cp, ri, v = [0], [], []
+    for j in range(nl + w):
+        if j < nl:
+            rows = np.concatenate([[j], nl + np.nonzero(V[:, j])[0]])
+            x = np.concatenate([[1.0], V[rows[1:] - nl, j]])
+        else:
+            rows, x = np.arange(j, nl + w), S[j - nl:, j - nl]
+        ri.append(rows)
+        v.append(x)
+        cp.append(cp[-1] + len(rows))
+    A = T.from_arrays(nl + w, np.array(cp), np.concatenate(ri), np.concatenate(v))
+    PA = T.permute(A, *T.order(A, "identity"))
+    T.lib.taucs_amd_set_solve_kernel(1 if chained else 0)
+    try:
+        F = T.factor_symbolic(PA)
+        assert F.numeric(PA, precision) == 0
+    finally:
+        T.lib.taucs_amd_set_solve_kernel(1)
+    sn, sched = F.supernodes(), F.schedule()
+    assert list(sn["sn_size"][sn["sn_size"] > 0]) == [1] * nl + [w]
+    parent = int(np.argmax(sn["sn_size"]))
+    order, c = [], int(sn["first_child"][parent])
+    while c != -1:
+        order.append(int(sn["struct_idx"][sn["struct_ptr"][c]]))
+        assert sched["level"][c] == 0 and sn["sn_up_size"][c] - 1 > 256
+        c = int(sn["next_child"][c])
+    assert sorted(order) == list(range(nl))
+    assert list(F.extend_adds(solve=True)["parents"]) == [3]
+    b = rng.uniform(-1, 1, (nl + w, nrhs)).astype(real).astype(np.float64)
+    x = b[nl:].astype(real)
+    for j in order:
+        x = x - V[:, j:j + 1].astype(real) * b[j].astype(real)
+    assert np.array_equal(F.solve(b)[nl:], x.astype(np.float64))
+    F.free()
