@@ -195,7 +195,11 @@ extern "C" void taucs_amd_set_panel_width(int w)
 }
 static int g_tile_big = 64;
 // With 128-tiles selected, a launch with fewer 128-tiles than this uses
-// 64-tiles instead (four times as many workgroups for the 256 CUs).
+// 64-tiles instead (four times as many workgroups): the line lies where the tiles
+// give each of the 256 CUs the two workgroups that it holds.  It is flat: steps with
+// 128, 256, 512 and 1024, ms: mesh3d 60^3 FP64 with 8 right-hand sides 26.20, 26.16,
+// 26.17, 26.08; 80^3 FP64 107.9, 108.2, 108.4, 108.1; 80 x 72 x 64 FP32 41.2, 41.2,
+// 41.1, 41.0; two runs of one side differ by 0.1 to 0.6%.
 #ifndef TILE128_MIN
 #define TILE128_MIN 512
 #endif
@@ -372,9 +376,6 @@ static double tile_flops(const GemmTask& g)
 
 static const int SMALL_M = 64;   // fronts with m <= 64 run whole in one wave
 static const int NB = 64;        // panel block width of large fronts
-// elements behind the L arena: k_gemm_tile128 loads 16 bytes from the last
-// row of a column on (3 elements past it in FP32, 1 in FP64)
-static const long long L_SPARE = 4;
 
 // One independent system of a (possibly batched) device schedule.
 struct SysView {
@@ -1305,10 +1306,17 @@ struct Emitter {
     if (E.kernel(__VA_ARGS__) != 0) return -1; \
   } while (0)
 
-// LDS per CU is 160 KiB.  Side-lane 64-tiles: FP64 two per CU (waves of 104
-// registers, leaving 304 on each SIMD and 52 KiB of LDS for a panel step's
-// workgroup: waves of 253 registers, 51 KiB); FP32 four per CU (64-register
-// waves, the panel step's 153 registers and 26 KiB).
+// LDS per CU is 160 KiB.  Side-lane 64-tiles: FP64 two per CU (waves of 106
+// registers, 112 allocated, leaving 288 on each SIMD and 52 KiB of LDS for a panel
+// step's workgroup: waves of 253 registers, 51 KiB); FP32 four per CU (76 registers,
+// 80 allocated, leaving 192 and 27 KiB for the panel step's 153 and 26 KiB).
+// In FP64 only while the update is short enough for the chain to be the longer
+// branch: a long update at half occupancy costs more than the overlap saves.
+// Factorizations, ms, with the reserve in no launch, in those of at most 4096 tiles, in
+// all: mesh3d 60^3 by 64-tiles 25.57, 24.84, 24.92, by 128-tiles (64 where a launch has
+// fewer than 512) 23.42, 23.14, 23.18; 80^3 by 64-tiles 126.2, 125.0, 126.5.  Where
+// the limit lies is flat: steps by 128-tiles with 2048, 4096 and 8192 26.14, 26.17,
+// 26.16 (60^3) and 108.1, 108.4, 108.2 (80^3).
 template <typename T> constexpr int SIDE_WGS = sizeof(T) == 8 ? 2 : 4;
 #define SIDE_PAD_MAX_TILES_FP64 4096
 #ifndef LAT_TILES_MAX
@@ -1399,7 +1407,10 @@ static int launch_numeric(tamd_dev* D, Emitter& E, bool bf16upd, bool prof)
         // the latency-shaped tile (the same bits) where each workgroup has a
         // CU to itself: K <= 64, or a main-chain launch of at most
         // LAT_TILES_MAX tiles (the next outer panel's columns of the top
-        // fronts: K = W in 4 round trips per 256 instead of 16)
+        // fronts: K = W in 4 round trips per 256 instead of 16; steps with a
+        // limit of 0 and 512: mesh3d 37 x 23 x 51 4.53 and 4.50 ms, 60^3 26.06 and
+        // 26.02; of 256, 512 and 1024: 60^3 26.18, 26.17, 26.15, 80^3 108.3, 108.4,
+        // 108.3)
         else if (lane == 0 && (op.shortk || op.count <= LAT_TILES_MAX))
           EMIT(lane, join, k_gemm_short<T>, dim3(op.count), dim3(256),
                (const GemmTask*)(D->d_gemm + op.start), (const T*)L, L, U, (const T*)Iv);
@@ -1407,11 +1418,7 @@ static int launch_numeric(tamd_dev* D, Emitter& E, bool bf16upd, bool prof)
           // The lookahead's trailing update reserves LDS it does not use, so
           // that at most SIDE_WGS<T> of its workgroups share a CU: the panel
           // chain's POTRF, TRSM and inner updates then find room beside it
-          // instead of waiting for the whole update to drain.  In FP64 only
-          // while the update is short enough for the chain to be the longer
-          // branch: a long update at half occupancy costs more than the
-          // overlap saves (measured: mesh3d 60^3 root, 2.3K tiles, gains 5%;
-          // 80^3 root, 20K tiles, loses 4%).
+          // instead of waiting for the whole update to drain.
           if (lane == 1 && (sizeof(T) == 4 || op.count <= SIDE_PAD_MAX_TILES_FP64))
             E.shmem = side_lds_pad<T>();
           EMIT(lane, join, k_gemm_tile<T>, dim3(op.count), dim3(256),

@@ -529,9 +529,9 @@ __global__ __launch_bounds__(64) void k_potrf_wave(const FrontDesc* __restrict__
 // last row is left.
 // L stays in the lower triangle; X, transposed, in the strict upper one
 // (X(r, c) at A[r*PM_LDA + c], r > c), its diagonal is rdiag.
-// Measured on one block, 64 columns, launch included: FP64 18.3 -> 11.9 us,
-// FP32 18.3 -> 15.3 us, against panels by one wave whose multipliers came by
-// readlane, and an inverse after the last panel.
+// One block of 64 columns alone on the card, the launch's time in the kernel trace
+// (median of 60): FP64 18.9 -> 12.6 us, FP32 19.7 -> 16.0 us, against panels by one
+// wave whose multipliers came by readlane, and an inverse after the last panel.
 // The MFMA steps apply their products as one fused multiply-add after another
 // in k order, so L and the inverse are bitwise those of k_potrf_wave.
 #define PM_LDA 65
@@ -1989,6 +1989,10 @@ __global__ __launch_bounds__(256) void k_panel_solve(const SolveTask* __restrict
       }
   // loader of a chunk: VEC rows from lr on, columns lk + 16 / NV * v
   const int lr = (tid % RG) * VEC, lk = tid / RG;
+  // (the last load of a column may pass its row M or N by VEC - 1 elements, at most
+  // L_SPARE past the arena: other rows' values, which end in rows and columns of the
+  // products that are not stored or become zero)
+  static_assert(VEC - 1 <= L_SPARE, "");
   const T* const Xr = L + t.xr_off + min(lr, t.M - 1) + lk * ld;
   const T* const Xk = L + t.xk_off + min(lr, t.N - 1) + lk * ld;
   T* const sA = As + lk * LDR + lr;
@@ -2252,6 +2256,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_tile128(const GemmTask* __restr
       for (int r = 0; r < 4; r++) acc[a][b][r] = (T)0;
 
   const int lr = (tid % RG) * VEC, lk = RG == 64 ? wave : tid / RG;
+  static_assert(VEC - 1 <= L_SPARE, "");
   const int lam = min(lr, t.M - 1), lbn = min(lr, t.N - 1), K1 = t.K - 1;
   vec_t ra[NQ], rb[NQ];
   T* const sA = As + lk * LDR + lr;

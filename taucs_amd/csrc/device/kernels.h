@@ -21,6 +21,11 @@ typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
+// Elements behind the L arena.  k_gemm_tile128 and k_panel_solve load 16 bytes from
+// the last row of a column on: up to 3 elements past it in FP32, 1 in FP64, and past
+// the arena after its last column.  (What is read there is dropped.)
+static const long long L_SPARE = 4;
+
 struct FrontDesc {
   long long offL;   // panel offset (elements)
   long long offU;   // update block offset
@@ -133,28 +138,6 @@ __device__ __forceinline__ void publish(T* p, T v)
   typedef typename Sentinel<T>::U U;
   __hip_atomic_store(reinterpret_cast<U*>(p), __builtin_bit_cast(U, v), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// one value, awaited (bounded: after SPIN_LIMIT polls the error word is marked
-// and the pattern is returned as it is; once any wait of the launch has marked
-// the error word, every other wait gives up at its next poll)
-template <typename T>
-__device__ __forceinline__ T await_value(const T* p, int* err)
-{
-  typedef typename Sentinel<T>::U U;
-  U* a = reinterpret_cast<U*>(const_cast<T*>(p));
-  U v = __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  int it = 0;
-  while (v == Sentinel<T>::bits) {
-    if (++it > SPIN_LIMIT) {
-      atomicOr(err, 1);
-      break;
-    }
-    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-    __builtin_amdgcn_s_sleep(1);
-    v = __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  return __builtin_bit_cast(T, v);
 }
 
 // ---- launches ---------------------------------------------------------------

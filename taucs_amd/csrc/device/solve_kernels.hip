@@ -462,7 +462,8 @@ __global__ __launch_bounds__(256) void k_bwd_step(const FrontDesc* __restrict__ 
 // is running, so the smallest unfinished ticket can always proceed.  Every
 // wait is still bounded: after SPIN_LIMIT polls the value is taken as it is,
 // the error word is marked and the task finishes (the solve reports failure);
-// every other wait of the launch then gives up at its next poll.
+// every other wait of the launch gives up within its next 32 polls, when it looks at
+// the error word.
 // Launches whose tasks wait for nothing run with ticket == nullptr (task =
 // blockIdx).
 
@@ -623,9 +624,13 @@ __global__ void k_sweep_clear(T* __restrict__ Y, double* __restrict__ x, int n, 
 // Values loaded ahead stay in registers from here on (the compiler may otherwise
 // move their loads behind the waits, to their first use).  The chains hold the
 // block inverse's operands this way: staged in LDS they were read on the chain's
-// critical path, and their 33 KiB (FP64) left three workgroups a CU.  Solve of
-// mesh3d 40^3 with one right-hand side 1083 -> 992 us, of mesh3d 60^3 with eight
-// 3060 -> 2903.
+// critical path.  Resident workgroups did not grow with it: the 33 KiB of LDS (FP64)
+// had left three a CU; the registers now leave three for up to eight right-hand sides
+// (149 to 156) and two for nine to sixteen (175 and 169), and three instead of four
+// to FP32's forward chain of those.  Solves, us, one, eight, nine and sixteen
+// right-hand sides: FP64 mesh3d 40^3 1083 -> 992, 1414 -> 1292, 1703 -> 1555, 2036 ->
+// 1864; 60^3 with eight, nine and sixteen 3045 -> 2888, 3675 -> 3461, 4600 -> 4329; FP32
+// with sixteen 40^3 1670 -> 1500, 60^3 3789 -> 3415.
 template <typename T> __device__ __forceinline__ void pin(T (&v)[16])
 {
 #pragma unroll
@@ -977,7 +982,10 @@ __device__ __forceinline__ void wave_sync_lds()
 // (One at a time, a front waited for s + m round trips to memory, each for as
 // little as one fused multiply-add a lane: the backward launch of 42 thousand fronts
 // of an 80 x 72 x 64 grid, four right-hand sides, took 91 us, this way 60; of 54
-// thousand fronts of 512 planes, one right-hand side, 126 and 89.)
+// thousand fronts of 512 planes, one right-hand side, 124 and 87.  The largest
+// forward launch, the 512 planes' 210 thousand leaves, is bound by its loads and lost,
+// 284 and 305 us, for the masked entries that are now read too; the backward launch of
+// the same leaves went from 348 to 299, the whole solve from 3.07 to 2.85 ms.)
 template <typename T, int N> struct SmallRows {
   const T* a;
   int stride, lo, hi;
