@@ -699,7 +699,11 @@ __device__ __forceinline__ void pm_panel_diag(const T* A, T* rdiag, const T* dg,
   T rd;
   sqrt_pair(P, d, rd);
   if (lane < 16) rdiag[c0 + li] = rd;
-  bad = bad || __ballot(!(P > (T)0)) != 0;
+  // an infinite pivot turns what follows it into NaNs, and a later pivot tells; but
+  // the columns after it may all lie past the block's and in panels that are left out
+  bool no = !(P > (T)0);
+  if constexpr (sizeof(T) == 8) no = no || (P == (T)__builtin_inf() && c0 + li < 63);
+  bad = bad || __ballot(no) != 0;
   if constexpr (sizeof(T) == 4) grow = grow || __ballot(P < (T)GROW_TAU * dg[c0 + li]) != 0;
 }
 

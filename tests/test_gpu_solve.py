@@ -398,3 +398,23 @@ def test_extend_adds_of_a_wide_parent_in_order(chained, precision, real):
         x = x - V[:, j:j + 1].astype(real) * b[j].astype(real)
     assert np.array_equal(F.solve(b)[nl:], x.astype(np.float64))
     F.free()
+
+
+@pytest.mark.parametrize("kb", [1, 15, 16, 17, 32, 33, 48, 63])
+def test_infinite_last_pivot_is_refused(kb):
+    """An infinite diagonal entry in the last column of an FP64 diagonal block of
+    fewer than 64 columns is a breakdown, whether or not the block ends with one
+    of its 16-column panels; the same entry made finite is not."""
+    print(f"case: infinite last pivot, dense {64 + kb}", flush=True)
+    n = 64 + kb
+    G = np.random.default_rng(n).standard_normal((n, n))
+    M = G @ G.T / n + 0.5 * np.eye(n)
+    i, j = np.triu_indices(n)
+    cp = np.concatenate([[0], np.cumsum(np.arange(n, 0, -1))])
+    for last, refused in ((np.inf, True), (1e300, False)):
+        M[n - 1, n - 1] = last
+        A = T.from_arrays(n, cp, j, M[i, j])
+        PA = T.permute(A, *T.order(A, "identity"))
+        F = T.factor_symbolic(PA)
+        assert (F.numeric(PA, T.FP64) != 0) == refused
+        F.free()
